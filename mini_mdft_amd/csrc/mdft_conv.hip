@@ -22,6 +22,7 @@
 // the block -> pair map gives every XCD a contiguous range of pairs so that
 // neighbouring pairs share L2 lines.
 #include "mdft_conv.hpp"
+#include "mdft_oz_group.hpp"
 #include "mdft_proj.hpp"
 
 #include <hip/hip_ext.h>
@@ -1336,6 +1337,7 @@ ConvDevice::ConvDevice(int nx, int ny, int nz, double lx, double ly, double lz, 
                  "internal error: the pairs of a star differ in kz");
       }
     stars = upload(st);
+    group = star32 && OzGroup::serves(mmax, mrso, nstars);
   }
   kxyz = upload(k3);
   pairs = upload(packed);
@@ -1471,6 +1473,13 @@ void ConvDevice::oz_pass(cplx<T>* p, double chop_eps, hipStream_t s, int nbatch,
   throw_if(tab.ang.np > 4 * kWave, "the OZ kernel handles at most 256 projections");
   throw_if(nbatch < 1, "OZ pass: bad batch");
   const T* dt = dtable<T>(s);
+  if constexpr (std::is_same<T, float>::value) {
+    if (group) {
+      if (!oz_group) oz_group = std::make_unique<OzGroup>(tab, s);
+      oz_group->run(p, dt, chop_eps, nbatch, compact, s, ev0, ev1);
+      return;
+    }
+  }
   OzArgs<T> a = oz_args<T>(*this, chop_eps);
   a.nbatch = nbatch;
   a.pstride = a.N * nbatch;

@@ -4,6 +4,7 @@
 #include <memory>
 
 #include "mdft_fft.hpp"
+#include "mdft_oz_group.hpp"
 
 namespace mdft {
 
@@ -50,6 +51,10 @@ struct ConvDevice {
   bool star32 = false, star64 = false;
   mutable int* dent = nullptr;  // LDS places codes of the half d table's entries (star kernel)
   mutable int* ccode = nullptr;  // per projection: its compact channel (compact_codes)
+  // FP32: whether the group kernel (mdft_oz_group.hip) takes this grid instead
+  // of the star kernel, and its tables, built on first use
+  bool group = false;
+  mutable std::unique_ptr<OzGroup> oz_group;
   // row width of the padded d layout when the compile-time OZ kernel serves
   // this (mmax, mrso) (2 mmax + 1), else 0 (compact rows, generic kernel)
   int padw = 0;
