@@ -12,7 +12,13 @@
 // writes the other (radix-4/2/3/5 butterflies, a generic odd-prime DFT up to
 // 13), with the twiddles e^{-2 pi i t/n} read from an LDS copy of an FP64
 // host table.
+//
+// Two sets of kernels with the same arithmetic: those here take any length at
+// run time; those of mdft_fft_ct.hpp are compiled for each smooth length from 8
+// to 128 and serve every axis of such a length and every square plane of one
+// that fits in LDS.
 #include "mdft_fft.hpp"
+#include "mdft_fft_ct.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -22,82 +28,6 @@
 namespace mdft {
 
 namespace {
-
-constexpr int kFftThreads = 256;
-constexpr int kMaxRadix = 13;
-
-template <typename T>
-__device__ __forceinline__ cplx<T> twiddle(const cplx<T>* tw, int t, int sign) {
-  cplx<T> w = tw[t];
-  if (sign > 0) w.y = -w.y;
-  return w;
-}
-
-// x * w with one fused and one rounded product, written out so that every
-// kernel (run-time or compile-time stages, any tiling) rounds the same way
-// whatever the compiler would contract
-template <typename T>
-__device__ __forceinline__ cplx<T> tw_mul(cplx<T> x, cplx<T> w) {
-  return mkc<T>(fma(x.x, w.x, -(x.y * w.y)), fma(x.x, w.y, x.y * w.x));
-}
-
-// in-place DFT of R values; sign -1 forward, +1 backward
-template <typename T>
-__device__ __forceinline__ void dft_small(cplx<T>* v, int R, int sign, const cplx<T>* tw, int n) {
-  if (R == 2) {
-    cplx<T> a = v[0], b = v[1];
-    v[0] = cadd<T>(a, b);
-    v[1] = csub<T>(a, b);
-  } else if (R == 4) {
-    cplx<T> s02 = cadd<T>(v[0], v[2]), d02 = csub<T>(v[0], v[2]);
-    cplx<T> s13 = cadd<T>(v[1], v[3]), d13 = csub<T>(v[1], v[3]);
-    // W = e^{sign 2 pi i/4} = sign * i
-    cplx<T> wd = mkc<T>(-static_cast<T>(sign) * d13.y, static_cast<T>(sign) * d13.x);
-    v[0] = cadd<T>(s02, s13);
-    v[2] = csub<T>(s02, s13);
-    v[1] = cadd<T>(d02, wd);
-    v[3] = csub<T>(d02, wd);
-  } else if (R == 3) {
-#pragma clang fp contract(off)
-    const T h = static_cast<T>(0.86602540378443864676);  // sqrt(3)/2
-    cplx<T> a = v[0], t = cadd<T>(v[1], v[2]), u = csub<T>(v[1], v[2]);
-    cplx<T> m = mkc<T>(a.x - static_cast<T>(0.5) * t.x, a.y - static_cast<T>(0.5) * t.y);
-    // sign * i * h * u
-    cplx<T> r = mkc<T>(-static_cast<T>(sign) * h * u.y, static_cast<T>(sign) * h * u.x);
-    v[0] = cadd<T>(a, t);
-    v[1] = cadd<T>(m, r);
-    v[2] = csub<T>(m, r);
-  } else {
-    cplx<T> out[kMaxRadix];
-    const int step = n / R;
-    for (int s = 0; s < R; ++s) {
-      cplx<T> acc = v[0];
-      for (int r = 1; r < R; ++r) acc = cfma<T>(acc, v[r], twiddle<T>(tw, ((r * s) % R) * step, sign));
-      out[s] = acc;
-    }
-    for (int s = 0; s < R; ++s) v[s] = out[s];
-  }
-}
-
-// DFT of R values held in registers (R fixed at compile time)
-template <typename T, int R>
-__device__ __forceinline__ void dft_fixed(cplx<T> (&v)[R], int sign, const cplx<T>* tw, int n) {
-  if constexpr (R == 2 || R == 3 || R == 4) {
-    dft_small<T>(v, R, sign, tw, n);
-  } else {
-    cplx<T> out[R];
-    const int step = n / R;
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-      cplx<T> acc = v[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) acc = cfma<T>(acc, v[r], twiddle<T>(tw, ((r * s) % R) * step, sign));
-      out[s] = acc;
-    }
-#pragma unroll
-    for (int s = 0; s < R; ++s) v[s] = out[s];
-  }
-}
 
 // One Stockham stage (radix R, Ns = product of the earlier radices) over the
 // wvalid lines of a tile: butterfly j of a line reads x[j + r n/R], applies the
@@ -257,7 +187,6 @@ size_t plane_lds(int ny, int nz) {
 // 160 KB LDS (at least two blocks of 8 waves per CU); the tuner also tries it
 // up to the whole LDS
 constexpr size_t kPlaneLdsMax = 80 * 1024;
-constexpr size_t kLdsMax = 160 * 1024;
 
 // One block transforms a tile of W lines of length n.
 //   STRIDED = false: line l occupies data[l*n .. l*n+n); the tile is lines
@@ -342,210 +271,13 @@ __global__ __launch_bounds__(kFftThreads) void fft_axis_kernel(cplx<T>* __restri
   }
 }
 
-// Compile-time kernels for the lengths the grids of the served mixes use
-// (16, 32, 48, 64, 80, 96, 128), with the radix schedule of FftPlan1D (4s
-// first, then 2, 3, 5).  Each stage is stockham_stage_2d with the length,
-// strides, line count and thread count known at compile time, so the index
-// arithmetic reduces to shifts, masks and constant divisions and the
-// butterfly loop unrolls; the arithmetic of every butterfly (LDS twiddles,
-// run-time sign, explicitly rounded products, operation order) is that of the
-// run-time stages, so results are bitwise the same.
-constexpr bool ct_length(int n) {
-  return n == 16 || n == 32 || n == 48 || n == 64 || n == 80 || n == 96 || n == 128;
-}
-template <int N>
-constexpr int ct_nstages() {
-  constexpr int ps[4] = {4, 2, 3, 5};
-  int r = N, c = 0;
-  for (int p : ps)
-    while (r % p == 0) {
-      r /= p;
-      ++c;
-    }
-  return c;
-}
-template <int N>
-constexpr int ct_radix(int s) {
-  constexpr int ps[4] = {4, 2, 3, 5};
-  int r = N, c = 0;
-  for (int p : ps)
-    while (r % p == 0) {
-      if (c == s) return p;
-      r /= p;
-      ++c;
-    }
-  return 0;
-}
-// the tile widths the FFT tuner tries for length N (values per tile 256,
-// 512, 1024, 2048; the default is the third)
-template <int N>
-constexpr int tuner_w(int i) {
-  constexpr int vals[4] = {256, 512, 1024, 2048};
-  const int w = vals[i] / N;
-  return w < 1 ? 1 : (w > 64 ? 64 : w);
-}
-
-template <typename T, int R, int N, int NS, int LS, int ES, int NLINES, int NTH, bool W_FAST>
-__device__ __forceinline__ void ct_stage_2d(const cplx<T>* src, cplx<T>* dst, const cplx<T>* tw, int sign, int tid) {
-  constexpr int NB = N / R, TSTEP = N / (NS * R), TOTAL = NLINES * NB;
-  constexpr int ITERS = (TOTAL + NTH - 1) / NTH;
-#pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    const int beta = tid + i * NTH;
-    if (TOTAL % NTH == 0 || beta < TOTAL) {
-      int w, j;
-      if constexpr (W_FAST) {
-        j = beta / NLINES;
-        w = beta - j * NLINES;
-      } else {
-        w = beta / NB;
-        j = beta - w * NB;
-      }
-      const int k = j % NS;
-      const cplx<T>* in = src + w * LS + j * ES;
-      cplx<T> v[R];
-      v[0] = in[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = tw_mul<T>(in[r * NB * ES], twiddle<T>(tw, r * k * TSTEP, sign));
-      dft_fixed<T, R>(v, sign, tw, N);
-      cplx<T>* out = dst + w * LS + ((j / NS) * NS * R + k) * ES;
-#pragma unroll
-      for (int r = 0; r < R; ++r) out[r * NS * ES] = v[r];
-    }
-  }
-}
-
-// stages S.. of one axis over an LDS tile, ping-pong between a and b; the
-// result ends in a when the remaining stage count is even, else in b
-template <typename T, int N, int LS, int ES, int NLINES, int NTH, bool W_FAST, int S = 0, int NS = 1>
-__device__ __forceinline__ void ct_stockham_2d(cplx<T>* a, cplx<T>* b, const cplx<T>* tw, int sign, int tid) {
-  if constexpr (S < ct_nstages<N>()) {
-    constexpr int R = ct_radix<N>(S);
-    ct_stage_2d<T, R, N, NS, LS, ES, NLINES, NTH, W_FAST>(a, b, tw, sign, tid);
-    __syncthreads();
-    ct_stockham_2d<T, N, LS, ES, NLINES, NTH, W_FAST, S + 1, NS * R>(b, a, tw, sign, tid);
-  }
-}
-
-// fft_plane_kernel for an N x N plane with NTH threads
-template <typename T, int N, int NTH>
-__global__ __launch_bounds__(NTH) void fft_plane_ct_kernel(cplx<T>* __restrict__ data, const cplx<T>* __restrict__ twz_g,
-                                                           const cplx<T>* __restrict__ twy_g, int sign) {
-  extern __shared__ unsigned char lds_raw[];
-  constexpr int LD = N + 1, NN = N * N, ITERS = (NN + NTH - 1) / NTH;
-  cplx<T>* bufA = reinterpret_cast<cplx<T>*>(lds_raw);
-  cplx<T>* bufB = bufA + N * LD;
-  cplx<T>* twz = bufB + N * LD;
-  cplx<T>* twy = twz + N;
-  const int tid = threadIdx.x;
-  if (tid < N) {
-    twz[tid] = twz_g[tid];
-    twy[tid] = twy_g[tid];
-  }
-  cplx<T>* plane = data + static_cast<long>(blockIdx.x) * NN;
-#pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    const int t = tid + i * NTH;
-    if (NN % NTH == 0 || t < NN) bufA[(t / N) * LD + t % N] = plane[t];
-  }
-  __syncthreads();
-  // z along the rows, then y along the columns
-  ct_stockham_2d<T, N, LD, 1, N, NTH, false>(bufA, bufB, twz, sign, tid);
-  constexpr bool z_in_a = ct_nstages<N>() % 2 == 0;
-  cplx<T>* a = z_in_a ? bufA : bufB;
-  cplx<T>* b = z_in_a ? bufB : bufA;
-  ct_stockham_2d<T, N, 1, LD, N, NTH, true>(a, b, twy, sign, tid);
-  const cplx<T>* res = bufA;  // two axes of the same stage count end where they began
-#pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    const int t = tid + i * NTH;
-    if (NN % NTH == 0 || t < NN) plane[t] = res[(t / N) * LD + t % N];
-  }
-}
-
-// fft_axis_kernel for length N and full tiles of W lines (W one of the tuner's widths)
-template <typename T, bool STRIDED, int N, int W>
-__global__ __launch_bounds__(kFftThreads) void fft_axis_ct_kernel(cplx<T>* __restrict__ data,
-                                                                  const cplx<T>* __restrict__ tw_g, int sign, long S) {
-  extern __shared__ unsigned char lds_raw[];
-  constexpr int LD = N + 1, NTH = kFftThreads, WN = W * N, ITERS = (WN + NTH - 1) / NTH;
-  cplx<T>* bufA = reinterpret_cast<cplx<T>*>(lds_raw);
-  cplx<T>* bufB = bufA + W * LD;
-  cplx<T>* tw = bufB + W * LD;
-  const int tid = threadIdx.x;
-  if (tid < N) tw[tid] = tw_g[tid];
-  long base;
-  if constexpr (!STRIDED) {
-    base = static_cast<long>(blockIdx.x) * (W * N);
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      if (WN % NTH == 0 || t < WN) bufA[(t / N) * LD + t % N] = data[base + t];
-    }
-  } else {
-    const long nchunk = S / W;
-    const long o = blockIdx.x / nchunk;
-    base = o * N * S + (blockIdx.x - o * nchunk) * W;
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      const int e = t / W, w = t % W;
-      if (WN % NTH == 0 || t < WN) bufA[w * LD + e] = data[base + static_cast<long>(e) * S + w];
-    }
-  }
-  __syncthreads();
-  ct_stockham_2d<T, N, LD, 1, W, NTH, false>(bufA, bufB, tw, sign, tid);
-  const cplx<T>* res = ct_nstages<N>() % 2 == 0 ? bufA : bufB;
-  if constexpr (!STRIDED) {
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      if (WN % NTH == 0 || t < WN) data[base + t] = res[(t / N) * LD + t % N];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      const int e = t / W, w = t % W;
-      if (WN % NTH == 0 || t < WN) data[base + static_cast<long>(e) * S + w] = res[w * LD + e];
-    }
-  }
-}
-
-// the compile-time kernel of (n, W), if any: f(integral_constant N, W)
-template <typename F>
-bool dispatch_axis_ct(int n, int W, F&& f) {
-  auto by_w = [&](auto nn) {
-    constexpr int N = decltype(nn)::value;
-    if (W == tuner_w<N>(0)) f(nn, std::integral_constant<int, tuner_w<N>(0)>{});
-    else if (W == tuner_w<N>(1)) f(nn, std::integral_constant<int, tuner_w<N>(1)>{});
-    else if (W == tuner_w<N>(2)) f(nn, std::integral_constant<int, tuner_w<N>(2)>{});
-    else if (W == tuner_w<N>(3)) f(nn, std::integral_constant<int, tuner_w<N>(3)>{});
-    else return false;
-    return true;
-  };
-  switch (n) {
-    case 16: return by_w(std::integral_constant<int, 16>{});
-    case 32: return by_w(std::integral_constant<int, 32>{});
-    case 48: return by_w(std::integral_constant<int, 48>{});
-    case 64: return by_w(std::integral_constant<int, 64>{});
-    case 80: return by_w(std::integral_constant<int, 80>{});
-    case 96: return by_w(std::integral_constant<int, 96>{});
-    case 128: return by_w(std::integral_constant<int, 128>{});
-    default: return false;
-  }
-}
-
-int choose_tile_lines(int n) {
+// default tile: a compiled width where there is one, else about 1024 values
+int choose_tile_lines(int n, bool strided) {
+  if (ct_length(n)) return strided ? 16 : contiguous_lines(n);
   int W = 1024 / n;
   if (W < 1) W = 1;
   if (W > 64) W = 64;
   return W;
-}
-
-template <typename T>
-size_t axis_lds(int n, int W) {
-  return (2 * static_cast<size_t>(W) * (n + 1) + n) * sizeof(cplx<T>);
 }
 
 template <typename T>
@@ -554,61 +286,26 @@ void launch_plane(cplx<T>* data, const FftPlan1D& pz, const FftPlan1D& py, long 
   const int n = pz.st.n;
   const size_t lds = plane_lds<T>(py.st.n, n);
   const dim3 grid(static_cast<unsigned>(planes));
-  if (py.st.n == n && ct_length(n) && n <= 96) {
-    auto go = [&](auto nn) {
-      constexpr int N = decltype(nn)::value;
-      if (threads == 256) {
-        hipLaunchKernelGGL((fft_plane_ct_kernel<T, N, 256>), grid, dim3(256), lds, s, data, pz.twiddles<T>(),
-                           py.twiddles<T>(), sign);
-      } else {
-        hipLaunchKernelGGL((fft_plane_ct_kernel<T, N, 512>), grid, dim3(512), lds, s, data, pz.twiddles<T>(),
-                           py.twiddles<T>(), sign);
-      }
-    };
-    switch (n) {
-      case 16: go(std::integral_constant<int, 16>{}); break;
-      case 32: go(std::integral_constant<int, 32>{}); break;
-      case 48: go(std::integral_constant<int, 48>{}); break;
-      case 64: go(std::integral_constant<int, 64>{}); break;
-      case 80: go(std::integral_constant<int, 80>{}); break;
-      default: go(std::integral_constant<int, 96>{}); break;
-    }
-  } else {
+  if (py.st.n != n || !launch_plane_ct<T>(data, pz.twiddles<T>(), n, planes, threads, sign, s)) {
     hipLaunchKernelGGL((fft_plane_kernel<T>), grid, dim3(threads), lds, s, data, pz.st, py.st, pz.twiddles<T>(),
                        py.twiddles<T>(), sign);
   }
   MDFT_HIP_CHECK(hipGetLastError());
 }
 
-// W = 0: the default tile (1024 / n lines)
+// W = 0: the default tile.  A compiled strided tile may be wider than the
+// stride as long as half of its columns exist (the missing ones are computed on
+// for nothing); with fewer, the run-time kernel takes a tile of the S columns.
 template <typename T>
 void launch_axis(cplx<T>* data, const FftPlan1D& p, int sign, long nlines_or_outer, long S, bool strided,
                  hipStream_t stream, int W = 0) {
   if (p.st.n == 1 || nlines_or_outer == 0) return;
-  if (W <= 0) W = choose_tile_lines(p.st.n);
-  if (strided && S < W) W = static_cast<int>(S);
+  if (W <= 0) W = choose_tile_lines(p.st.n, strided);
+  if (strided && S < W && !(ct_length(p.st.n) && strided_lines(W) && 2 * S >= W)) W = static_cast<int>(S);
   const size_t lds = axis_lds<T>(p.st.n, W);
   throw_if(lds > kLdsMax, "FFT tile does not fit in LDS");
   const cplx<T>* tw = p.twiddles<T>();
-  const bool full = strided ? S % W == 0 : nlines_or_outer % W == 0;
-  if (full && ct_length(p.st.n)) {
-    const long nblk = strided ? nlines_or_outer * (S / W) : nlines_or_outer / W;
-    throw_if(nblk > 0x7fffffffL, "too many FFT tiles");
-    const bool done = dispatch_axis_ct(p.st.n, W, [&](auto nn, auto ww) {
-      constexpr int N = decltype(nn)::value, WW = decltype(ww)::value;
-      if (strided) {
-        hipLaunchKernelGGL((fft_axis_ct_kernel<T, true, N, WW>), dim3(static_cast<unsigned>(nblk)), dim3(kFftThreads),
-                           lds, stream, data, tw, sign, S);
-      } else {
-        hipLaunchKernelGGL((fft_axis_ct_kernel<T, false, N, WW>), dim3(static_cast<unsigned>(nblk)),
-                           dim3(kFftThreads), lds, stream, data, tw, sign, S);
-      }
-    });
-    if (done) {
-      MDFT_HIP_CHECK(hipGetLastError());
-      return;
-    }
-  }
+  if (launch_axis_ct<T>(data, tw, p.st.n, W, strided, sign, nlines_or_outer, S, stream)) return;
   if (!strided) {
     const long nblk = (nlines_or_outer + W - 1) / W;
     throw_if(nblk > 0x7fffffffL, "too many FFT tiles");
@@ -672,7 +369,9 @@ Fft3dPlan::Fft3dPlan(int nx_, int ny_, int nz_) : nx(nx_), ny(ny_), nz(nz_), px(
 
 bool Fft3dPlan::plane_ok(size_t elem, int threads) const {
   (void)threads;
-  return ny > 1 && nz > 1 && small_radices(py.st) && small_radices(pz.st) &&
+  // the run-time plane kernel has radices up to 5; square planes of the
+  // compiled lengths have their own
+  return ny > 1 && nz > 1 && ((small_radices(py.st) && small_radices(pz.st)) || (ny == nz && plane_ct(ny, elem))) &&
          (2 * static_cast<size_t>(ny) * (nz + 1) + ny + nz) * elem <= kLdsMax;
 }
 
@@ -709,8 +408,9 @@ void Fft3dPlan::execute(cplx<T>* data, long batch, int sign, hipStream_t stream)
 }
 
 // Times the candidate configurations on a scratch array of `batch`
-// transforms and keeps the fastest: the tile width of each per-axis pass
-// (256, 512, 1024, 2048 values per tile) and, where a (y, z) plane fits in
+// transforms and keeps the fastest: the tile width of each per-axis pass (16 or
+// 32 columns of the compiled kernels, 256, 512, 1024 or 2048 values per tile of
+// the run-time ones) and, where a (y, z) plane fits in
 // LDS, the fused z/y pass with 256 or 512 threads.  Every candidate runs the
 // same Stockham stages on the same lines, so the choice changes timing only.
 template <typename T>
@@ -743,13 +443,20 @@ FftConfig Fft3dPlan::autotune(long batch, hipStream_t s) const {
       return best_ms;
     };
     const long nxl = nx, nyl = ny, nzl = nz;
-    // per-axis tile widths
+    // per-axis tile widths: the compiled ones, else tiles of 256 .. 2048 values
+    auto candidates = [](int n, long S, bool strided) {
+      if (ct_length(n)) return strided ? std::vector<int>{16, 32} : std::vector<int>{contiguous_lines(n)};
+      std::vector<int> w;
+      for (int vals : {256, 512, 1024, 2048}) {
+        w.push_back(std::max(1, std::min(64, vals / std::max(1, n))));
+        if (strided && S < w.back()) w.back() = static_cast<int>(S);
+      }
+      return w;
+    };
     auto best_w = [&](const FftPlan1D& p, long lines, long S, bool strided) {
       int bw = 0;
       float bt = 1e30f;
-      for (int vals : {256, 512, 1024, 2048}) {
-        int W = std::max(1, std::min(64, vals / std::max(1, p.st.n)));
-        if (strided && S < W) W = static_cast<int>(S);
+      for (int W : candidates(p.st.n, S, strided)) {
         if (axis_lds<T>(p.st.n, W) > kLdsMax) continue;
         const float t = time_ms([&] { launch_axis<T>(buf, p, -1, lines, S, strided, s, W); });
         if (t < bt) {
