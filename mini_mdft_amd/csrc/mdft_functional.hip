@@ -231,10 +231,15 @@ struct VextArgs {
 // minimum-image distance between solvent site k of orientation o at node r
 // and solute site j, floored at 1e-6 A; pair[(k nsolute + j) * 3] =
 // (sigma, 4 eps, qfact q q), sigma = 0 where either site has no LJ.  1/d is
-// one rsqrt of d^2, clamped at 1e6 (the floor): against a square root and a
-// division, 8.4 -> 5.3 ms at 64^3 / mmax 5 with 20 x 3 site pairs.  Sites at
+// one reciprocal root of d^2, clamped at 1e6 (the floor).  Sites at
 // the molecular origin are summed once per node (vext_node_kernel); when they
 // lead the site list, as the oxygen does, the sum keeps its order.
+
+// v + 4 eps ((sigma / d)^12 - (sigma / d)^6)
+__device__ __forceinline__ double lennard_jones(double sigma, double eps4, double inv, double v) {
+  const double sr = sigma * inv, sr2 = sr * sr, sr6 = sr2 * (sr2 * sr2);
+  return fma(eps4, fma(sr6, sr6, -sr6), v);
+}
 
 // v += sum_j [LJ_kj(d) + qq_kj / d] for solvent site k at (px, py, pz)
 __device__ __forceinline__ void vext_site(const VextArgs& a, double px, double py, double pz, int k,
@@ -247,10 +252,7 @@ __device__ __forceinline__ void vext_site(const VextArgs& a, double px, double p
     ddz -= a.lz * rint(ddz * a.ilz);
     const double inv = fmin(rsqrt(ddx * ddx + ddy * ddy + ddz * ddz), 1e6);
     const double* pp = pair + (static_cast<long>(k) * a.nsolute + j) * 3;
-    if (pp[0] > 0.0) {
-      const double sr = pp[0] * inv, sr2 = sr * sr, sr6 = sr2 * sr2 * sr2;
-      v += pp[1] * (sr6 * sr6 - sr6);
-    }
+    if (pp[0] > 0.0) v = lennard_jones(pp[0], pp[1], inv, v);
     v += pp[2] * inv;
   }
 }
@@ -283,24 +285,111 @@ __global__ __launch_bounds__(kFThreads) void vext_node_kernel(VextArgs a, unsign
   }
 }
 
-// V(r, o): Vr(r) (or 0 without origin sites), then the other sites in order
+// node coordinate plus site offset, both operations rounded
+__device__ __forceinline__ double site_coordinate(int i, double h, double o) {
+#pragma clang fp contract(off)
+  return i * h + o;
+}
+
+// min(1 / d, 1e6) from d^2.  BOUNDED (d^2 < inf): the hardware's estimate y and
+// one third-order step, y (1 - e)^(-1/2) = y (1 + e/2 + 3 e^2 / 8 + ..) with
+// e = 1 - d^2 y^2 (d = 0: NaN, which the minimum takes to 1e6).  Against
+// rsqrt(), which also selects for 0 and infinity: 2167 -> 1927 us at 64^3 / mmax
+// 5 with 20 x 2 pairs, the same bits.
+template <bool BOUNDED>
+__device__ __forceinline__ double inverse_distance(double d2) {
+  if constexpr (!BOUNDED) return fmin(rsqrt(d2), 1e6);
+  const double y = __builtin_amdgcn_rsq(d2);
+  const double e = fma(-d2 * y, y, 1.0);
+  return fmin(fma(y * e, fma(e, 0.375, 0.5), y), 1e6);
+}
+
+// V(r, o): Vr(r) (or 0 without origin sites), then the other sites in order.
+// One thread takes one orientation at a tile of TY x TZ nodes of an x row.
+// FP64 arithmetic bounds it, and a pair alone costs 31 vector operations, 15 of
+// them the minimum image and 10 the reciprocal root; the tile shares the x term
+// of d^2 over its nodes, the y terms over its columns and the z terms over its
+// rows, so that a pair has one addition and the root left.  A call at 64^3 /
+// mmax 5 with 20 x 2 pairs: one node 3228 us, 2 x 2 2309, 2 x 4 2006, 4 x 4 1927,
+// 4 x 8 (256 registers, one wave per SIMD) slower again.  The sums are the ones
+// vext_site makes, product for product.  Missing nodes of a ragged tile
+// repeat the last node and are not stored.
+template <int TY, int TZ, bool BOUNDED>
 __global__ __launch_bounds__(kFThreads) void vext_kernel(VextArgs a, unsigned origin, const double* __restrict__ Vr,
                                                          const double* __restrict__ off,
                                                          const double* __restrict__ pair,
                                                          const double* __restrict__ solute, double* __restrict__ V) {
-  for (long idx = static_cast<long>(blockIdx.x) * kFThreads + threadIdx.x; idx < a.n;
+  const int ny = a.nyz / a.nz, nty = (ny + TY - 1) / TY, ntz = (a.nz + TZ - 1) / TZ;
+  const long total = a.n / a.no / a.nyz * nty * ntz * a.no;
+  for (long idx = static_cast<long>(blockIdx.x) * kFThreads + threadIdx.x; idx < total;
        idx += static_cast<long>(gridDim.x) * kFThreads) {
-    const long r = idx / a.no;
-    const int io = static_cast<int>(idx - r * a.no);
-    double gx, gy, gz;
-    node_position(a, r, gx, gy, gz);
-    double v = Vr ? Vr[r] : 0.0;
+    const long tile = idx / a.no;
+    const int io = static_cast<int>(idx - tile * a.no);
+    const long row = tile / ntz;
+    const int z0 = static_cast<int>(tile - row * ntz) * TZ;
+    const int ix = static_cast<int>(row / nty);
+    const int y0 = static_cast<int>(row - static_cast<long>(ix) * nty) * TY;
+    int iy[TY], iz[TZ];
+    double v[TY][TZ];
+#pragma unroll
+    for (int y = 0; y < TY; ++y) iy[y] = min(y0 + y, ny - 1);
+#pragma unroll
+    for (int z = 0; z < TZ; ++z) iz[z] = min(z0 + z, a.nz - 1);
+#pragma unroll
+    for (int y = 0; y < TY; ++y)
+#pragma unroll
+      for (int z = 0; z < TZ; ++z)
+        v[y][z] = Vr ? Vr[static_cast<long>(ix) * a.nyz + static_cast<long>(iy[y]) * a.nz + iz[z]] : 0.0;
     for (int k = 0; k < a.nsolv; ++k) {
       if ((origin >> k) & 1u) continue;
       const double* o = off + (static_cast<long>(io) * a.nsolv + k) * 3;
-      vext_site(a, gx + o[0], gy + o[1], gz + o[2], k, pair, solute, v);
+      const double px = site_coordinate(ix, a.dx, o[0]);
+      double py[TY], pz[TZ];
+#pragma unroll
+      for (int y = 0; y < TY; ++y) py[y] = site_coordinate(iy[y], a.dy, o[1]);
+#pragma unroll
+      for (int z = 0; z < TZ; ++z) pz[z] = site_coordinate(iz[z], a.dz, o[2]);
+      for (int j = 0; j < a.nsolute; ++j) {
+        const double* pp = pair + (static_cast<long>(k) * a.nsolute + j) * 3;
+        const double sigma = pp[0], eps4 = pp[1], qq = pp[2];
+        double dx = px - solute[3 * j];
+        dx = fma(-a.lx, rint(dx * a.ilx), dx);
+        double xy[TY], dz[TZ];
+#pragma unroll
+        for (int y = 0; y < TY; ++y) {
+          double dy = py[y] - solute[3 * j + 1];
+          dy = fma(-a.ly, rint(dy * a.ily), dy);
+          xy[y] = fma(dx, dx, dy * dy);
+        }
+#pragma unroll
+        for (int z = 0; z < TZ; ++z) {
+          dz[z] = pz[z] - solute[3 * j + 2];
+          dz[z] = fma(-a.lz, rint(dz[z] * a.ilz), dz[z]);
+        }
+        if (sigma > 0.0) {
+#pragma unroll
+          for (int y = 0; y < TY; ++y)
+#pragma unroll
+            for (int z = 0; z < TZ; ++z) {
+              const double inv = inverse_distance<BOUNDED>(fma(dz[z], dz[z], xy[y]));
+              v[y][z] = fma(qq, inv, lennard_jones(sigma, eps4, inv, v[y][z]));
+            }
+        } else {
+#pragma unroll
+          for (int y = 0; y < TY; ++y)
+#pragma unroll
+            for (int z = 0; z < TZ; ++z)
+              v[y][z] = fma(qq, inverse_distance<BOUNDED>(fma(dz[z], dz[z], xy[y])), v[y][z]);
+        }
+      }
     }
-    V[idx] = fmin(v, a.vmax);
+#pragma unroll
+    for (int y = 0; y < TY; ++y)
+#pragma unroll
+      for (int z = 0; z < TZ; ++z)
+        if (y0 + y < ny && z0 + z < a.nz)
+          V[(static_cast<long>(ix) * a.nyz + static_cast<long>(iy[y]) * a.nz + iz[z]) * a.no + io] =
+              fmin(v[y][z], a.vmax);
   }
 }
 
@@ -376,19 +465,19 @@ void compute_vext(int nx, int ny, int nz, double lx, double ly, double lz, const
       p[2] = kQfact * qk * qj;
     }
   const long n = static_cast<long>(nx) * ny * nz * g.no;
-  // one-time tables: plain allocations, freed on every exit path
+  // one-time tables in one allocation (off, pair, pos, then Vr), freed on every
+  // exit path: a call on a small grid is mostly these (8^3, mmax 3: 62 us with
+  // four, 53 with one)
+  std::vector<double> host(off);
+  host.insert(host.end(), pair.begin(), pair.end());
+  host.insert(host.end(), pos.begin(), pos.end());
+  const long nr = static_cast<long>(nx) * ny * nz;
   struct Buf {
     double* p = nullptr;
     ~Buf() {
       if (p) (void)hipFree(p);
     }
-  } doff, dpair, dpos, dvr;
-  MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&doff.p), off.size() * sizeof(double)));
-  MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&dpair.p), pair.size() * sizeof(double)));
-  MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&dpos.p), pos.size() * sizeof(double)));
-  MDFT_HIP_CHECK(hipMemcpyAsync(doff.p, off.data(), off.size() * sizeof(double), hipMemcpyHostToDevice, s));
-  MDFT_HIP_CHECK(hipMemcpyAsync(dpair.p, pair.data(), pair.size() * sizeof(double), hipMemcpyHostToDevice, s));
-  MDFT_HIP_CHECK(hipMemcpyAsync(dpos.p, pos.data(), pos.size() * sizeof(double), hipMemcpyHostToDevice, s));
+  } tables;
   VextArgs a{n, g.no, ny * nz, nz, nsolvent, nsolute, lx / nx, ly / ny, lz / nz, lx, ly, lz,
              1.0 / lx, 1.0 / ly, 1.0 / lz, vmax};
   // solvent sites at the molecular origin (all of the site's offsets zero)
@@ -396,15 +485,34 @@ void compute_vext(int nx, int ny, int nz, double lx, double ly, double lz, const
   if (nsolvent <= 32)
     for (int k = 0; k < nsolvent; ++k)
       if (solvent[6 * k + 3] == 0.0 && solvent[6 * k + 4] == 0.0 && solvent[6 * k + 5] == 0.0) origin |= 1u << k;
-  const long nr = static_cast<long>(nx) * ny * nz;
+  MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&tables.p), (host.size() + (origin ? nr : 0)) * sizeof(double)));
+  MDFT_HIP_CHECK(hipMemcpyAsync(tables.p, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice, s));
+  const double *doff = tables.p, *dpair = doff + off.size(), *dpos = dpair + pair.size();
+  double* dvr = origin ? tables.p + host.size() : nullptr;
   if (origin) {
-    MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&dvr.p), nr * sizeof(double)));
-    hipLaunchKernelGGL(vext_node_kernel, dim3(grid_for(nr, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin,
-                       dpair.p, dpos.p, dvr.p);
+    hipLaunchKernelGGL(vext_node_kernel, dim3(grid_for(nr, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin, dpair,
+                       dpos, dvr);
     MDFT_HIP_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(vext_kernel, dim3(grid_for(n, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin, dvr.p,
-                     doff.p, dpair.p, dpos.p, vext);
+  auto launch = [&](auto kernel, int ty, int tz) {
+    const long threads = static_cast<long>(nx) * ((ny + ty - 1) / ty) * ((nz + tz - 1) / tz) * g.no;
+    hipLaunchKernelGGL(kernel, dim3(grid_for(threads, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin, dvr,
+                       doff, dpair, dpos, vext);
+  };
+  // 16 nodes per thread where that leaves every CU a block, else 4 (16^3, mmax
+  // 4, 58k against 230k threads: 117 and 115 us a call; 30 x 42 x 27, mmax 3,
+  // 191k: 102 and 109).  inverse_distance needs a finite d^2; coordinates that
+  // could overflow it keep the library's root.
+  auto bounded = [](const double* v, size_t count) {
+    return std::all_of(v, v + count, [](double x) { return std::abs(x) <= 1e100; });
+  };
+  const double box[3] = {lx, ly, lz};
+  if (!bounded(box, 3) || !bounded(pos.data(), pos.size()) || !bounded(off.data(), off.size()))
+    launch(vext_kernel<2, 2, false>, 2, 2);
+  else if (n / 16 < 65536)
+    launch(vext_kernel<2, 2, true>, 2, 2);
+  else
+    launch(vext_kernel<4, 4, true>, 4, 4);
   MDFT_HIP_CHECK(hipGetLastError());
   // the tables (host and device) are released on return
   MDFT_HIP_CHECK(hipStreamSynchronize(s));
