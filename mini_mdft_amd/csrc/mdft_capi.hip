@@ -277,11 +277,11 @@ int mdft_angl2proj(mdft_opt_t h, const void* o, void* p, void* stream) {
     switch (h->precision) {
       case MDFT_FP64:
         angl2proj_factorized<double, double, double>(*h->tab, h->N, static_cast<const double*>(o),
-                                                     static_cast<cplx<double>*>(p), nullptr, s);
+                                                     static_cast<cplx<double>*>(p), nullptr, s, false, h->N);
         break;
       case MDFT_FP32:
         angl2proj_factorized<float, float, float>(*h->tab, h->N, static_cast<const float*>(o),
-                                                  static_cast<cplx<float>*>(p), nullptr, s);
+                                                  static_cast<cplx<float>*>(p), nullptr, s, false, h->N);
         break;
       case MDFT_MIXED_X6F:
         h->gemm->angl2proj(h->N, static_cast<const float*>(o), static_cast<cplx<float>*>(p), nullptr, s);
@@ -633,7 +633,7 @@ static void energy_impl(mdft_solver_t h, int nb, const void* xi, void* df, doubl
     case MDFT_FP64: {
       auto* p = static_cast<cplx<double>*>(h->pbuf);
       angl2proj_factorized<double, double, double>(*h->tab, Nb, static_cast<const double*>(xi), p, &rho0, s,
-                                                   h->compact);
+                                                   h->compact, h->N);
       h->conv->dev->execute<double>(p, eps, s, tm, nb, h->compact);
       proj2angl_factorized<double, double, double>(*h->tab, Nb, p, nullptr, static_cast<const double*>(xi),
                                                    static_cast<double*>(df), rho0, h->partials, s, colp,
@@ -643,7 +643,7 @@ static void energy_impl(mdft_solver_t h, int nb, const void* xi, void* df, doubl
     case MDFT_FP32: {
       auto* p = static_cast<cplx<float>*>(h->pbuf);
       angl2proj_factorized<float, float, float>(*h->tab, Nb, static_cast<const float*>(xi), p, &rho0, s,
-                                                h->compact);
+                                                h->compact, h->N);
       h->conv->dev->execute<float>(p, eps, s, tm, nb, h->compact);
       proj2angl_factorized<float, float, float>(*h->tab, Nb, p, nullptr, static_cast<const float*>(xi),
                                                 static_cast<float*>(df), rho0, h->partials, s, colp,

@@ -19,7 +19,7 @@
 // Re of the DC bin and twice Re of the others (npsi = 2 mmax/mrso + 1 is odd,
 // so there is no Nyquist bin).  Optionally get_delta_f
 // (common/MDFT_Solvent.hpp:613-660) is fused into the last step.
-#include "mdft_proj.hpp"
+#include "mdft_proj_ct.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -33,15 +33,6 @@ constexpr int kRT = 8;  // r values per block
 
 struct TileDims {
   int ntheta, nphi, npsi, nmu2, no, np, mmax;
-};
-
-template <typename TC>
-struct TabPtrs {
-  const cplx<TC>* ephi;
-  const cplx<TC>* epsi;
-  const TC* wts;
-  const int* ipinfo;
-  const int* yidx;
 };
 
 __device__ __forceinline__ int pmod(int a, int n) {
@@ -142,20 +133,10 @@ __global__ __launch_bounds__(kThreads) void angl2proj_kernel(const TI* __restric
 
 // angl2proj_kernel for an angular grid fixed at compile time (the grids of
 // dispatch_angular): the same three steps with every extent a constant, so
-// that the index arithmetic folds and the short loops unroll.
-template <int MMAX, int MRSO, int RT>
-struct A2pSizes {
-  static constexpr int kNth = MMAX + 1, kNphi = 2 * MMAX + 1, kNmu2 = MMAX / MRSO + 1;
-  static constexpr int kNpsi = 2 * (MMAX / MRSO) + 1, kNo = kNth * kNphi * kNpsi;
-  static constexpr int kNp() {
-    int n = 0;
-    for (int m = 0; m <= MMAX; ++m) n += (2 * m + 1) * (m / MRSO + 1);
-    return n;
-  }
-  static constexpr int kCells = RT * kNth * kNphi * kNmu2;
-  static constexpr int kRegA = (2 * kCells > RT * kNo) ? 2 * kCells : RT * kNo;
-};
-
+// that the index arithmetic folds and the short loops unroll.  For fields of
+// few points (mdft_a2p_wave.hip has the others), where a block per 4 or 8 rows
+// reaches more of the chip: 12^3 mmax 5 FP64 12.5 us against 18.4, 16^3 mmax 4
+// 12.8 against 18.3.
 // rows per block of the compile-time angl2proj: 4 in FP64, whose tile holds
 // twice the bytes (more blocks per CU), 8 in FP32
 template <typename TC>
@@ -797,24 +778,6 @@ ProjTables::~ProjTables() {
 
 namespace {
 
-// the angular grids with a compile-time proj2angl kernel: mrso = 2 with mmax
-// 1..6 and mrso = 1 with mmax 1..3 (larger mrso = 1 grids hold too many S
-// registers per lane and take the generic kernel)
-template <int MMAX = 1, int MRSO = 1, typename F>
-bool dispatch_angular(int mmax, int mrso, F&& f) {
-  if constexpr (MMAX > 6) {
-    return false;
-  } else if constexpr (MRSO > 2 || (MRSO == 1 && MMAX > 3)) {
-    return dispatch_angular<MMAX + (MRSO > 2 ? 1 : 0), MRSO + (MRSO > 2 ? -2 : 1)>(mmax, mrso, f);
-  } else {
-    if (mmax == MMAX && mrso == MRSO) {
-      f(std::integral_constant<int, MMAX>{}, std::integral_constant<int, MRSO>{});
-      return true;
-    }
-    return dispatch_angular<MMAX, MRSO + 1>(mmax, mrso, f);
-  }
-}
-
 long wave_row_blocks(long N) { return (N + kWaveRows - 1) / kWaveRows; }
 
 long wave_blocks(const ProjTables& t, long N) {
@@ -826,10 +789,12 @@ long wave_blocks(const ProjTables& t, long N) {
 
 template <typename TI, typename TP, typename TC>
 void angl2proj_factorized(const ProjTables& t, long N, const TI* o, cplx<TP>* p, const double* drho_rho0,
-                          hipStream_t s, bool compact) {
+                          hipStream_t s, bool compact, long field) {
   if (N == 0) return;
   const long nblk = (N + kRT - 1) / kRT;
   throw_if(nblk > 0x7fffffffL, "grid too large");
+  if constexpr (std::is_same<TI, TC>::value)
+    if (launch_a2p_wave<TI, TP, TC>(t, N, field, o, p, tabs_of<TC>(t, true), drho_rho0, s, compact)) return;
   bool compiled = false;
   dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
     constexpr int MMAX = decltype(mm)::value, MRSO = decltype(mr)::value, RT = a2p_ct_rows<TC>();
@@ -962,11 +927,11 @@ void fill_uniform(T* x, size_t n, unsigned long long seed, unsigned long long of
 }
 
 template void angl2proj_factorized<double, double, double>(const ProjTables&, long, const double*, cplx<double>*,
-                                                           const double*, hipStream_t, bool);
+                                                           const double*, hipStream_t, bool, long);
 template void angl2proj_factorized<float, float, float>(const ProjTables&, long, const float*, cplx<float>*,
-                                                        const double*, hipStream_t, bool);
+                                                        const double*, hipStream_t, bool, long);
 template void angl2proj_factorized<double, float, float>(const ProjTables&, long, const double*, cplx<float>*,
-                                                         const double*, hipStream_t, bool);
+                                                         const double*, hipStream_t, bool, long);
 template void proj2angl_factorized<double, double, double>(const ProjTables&, long, const cplx<double>*, double*,
                                                            const double*, double*, double, double*, hipStream_t,
                                                            double*, bool);

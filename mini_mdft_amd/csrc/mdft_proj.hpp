@@ -93,9 +93,12 @@ std::vector<int> compact_codes(const AngularGrid& g);
 // formed on load (common/MDFT_Solvent.hpp:575-596 fused).
 // With compact, only the stored projections of the compact channel order are
 // written, at their compact channels (compile-time grids, angl2proj_compiled).
+// field: the points of one field of the N, by which the kernel is chosen, so
+// that a field has the same bits alone and in a batch (0: the kernel for few
+// points).
 template <typename TI, typename TP, typename TC>
 void angl2proj_factorized(const ProjTables& t, long N, const TI* o, cplx<TP>* p, const double* drho_rho0,
-                          hipStream_t s, bool compact = false);
+                          hipStream_t s, bool compact = false, long field = 0);
 // whether angl2proj_factorized has a compile-time kernel for this grid with
 // FP64 (fp64) or FP32 arithmetic
 bool angl2proj_compiled(const ProjTables& t, bool fp64);
