@@ -92,7 +92,7 @@ struct mdft_solver_s {
   void* pbuf = nullptr;  // projections, np x N complex (compact: the first channels)
   double* partials = nullptr;
   int nparts = 0;
-  double* ffdev = nullptr;
+  double* ffhost = nullptr;  // pinned: the reduction stores the energies here, no copy follows it
   size_t bytes = 0;
   std::unique_ptr<StageTimer> timer;  // set while stage timing is on
   // the r-mean (q = 0) mode of ff in FP64 (on by default for MDFT_MIXED_X6)
@@ -105,7 +105,7 @@ struct mdft_solver_s {
   ~mdft_solver_s() {
     if (pbuf) (void)hipFree(pbuf);
     if (partials) (void)hipFree(partials);
-    if (ffdev) (void)hipFree(ffdev);
+    if (ffhost) (void)hipHostFree(ffhost);
     if (colpart) (void)hipFree(colpart);
     if (meanwork) (void)hipFree(meanwork);
     if (extra) (void)hipFree(extra);
@@ -586,7 +586,7 @@ int mdft_solver_create_batch(mdft_conv_t conv, double rho0, double prefactor, in
     h->nparts = h->field_parts * capacity;
     MDFT_HIP_CHECK(hipMalloc(&h->pbuf, pbytes));
     MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&h->partials), h->nparts * sizeof(double)));
-    MDFT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&h->ffdev), capacity * sizeof(double)));
+    MDFT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h->ffhost), capacity * sizeof(double), 0));
     h->bytes = pbytes + (h->nparts + capacity) * sizeof(double);
     if ((precision == MDFT_MIXED_X6 || precision == MDFT_MIXED_X6F) && mean_mode_supported(h.get())) {
       enable_mean_mode(h.get());
@@ -737,9 +737,11 @@ int mdft_energy_cproj_batch(mdft_solver_t h, int nbatch, const void* xi, void* d
   return guarded([&] {
     throw_if(!ff, "energy_cproj: null ff");
     hipStream_t s = as_stream(stream);
-    energy_impl(h, nbatch, xi, df, h ? h->ffdev : nullptr, 1, s);
-    MDFT_HIP_CHECK(hipMemcpyAsync(ff, h->ffdev, nbatch * sizeof(double), hipMemcpyDeviceToHost, s));
+    double* out = nullptr;
+    if (h) MDFT_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&out), h->ffhost, 0));
+    energy_impl(h, nbatch, xi, df, out, 1, s);
     MDFT_HIP_CHECK(hipStreamSynchronize(s));
+    std::copy(h->ffhost, h->ffhost + nbatch, ff);
   });
 }
 

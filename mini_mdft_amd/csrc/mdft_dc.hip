@@ -38,62 +38,71 @@ namespace mdft {
 
 namespace {
 
-// One reduction pass over the per-row-block column sums: out[j][c][col] =
-// sum of in[j][kFan c + i][col] over i < kFan (fixed order; rows past the
-// field's count read as zero).  One wave per (chunk c, 64 columns, field j),
-// all kFan loads of a thread in flight together.
+// The sum of column col of nin rows, rows c kFan .. (fixed order; rows past the
+// last read as zero), all kFan loads in flight together.
 constexpr int kFan = 64;
+__device__ __forceinline__ double column_sum(const double* __restrict__ src, long nin, int width, long c, int col) {
+  double v[kFan];
+#pragma unroll
+  for (int i = 0; i < kFan; ++i) v[i] = src[min(c * kFan + i, nin - 1) * width + col];
+#pragma unroll
+  for (int i = 0; i < kFan; ++i) v[i] = c * kFan + i < nin ? v[i] : 0.0;
+#pragma unroll
+  for (int h = kFan / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int i = 0; i < h; ++i) v[i] += v[i + h];
+  return v[0];
+}
+
+// One reduction pass over the per-row-block column sums: out[j][c][col] =
+// the sum of in[j][kFan c + i][col] over i < kFan.  One wave per (chunk c, 64
+// columns, field j).
 __global__ __launch_bounds__(64) void mean_colsum_kernel(const double* __restrict__ in, long nin, int width,
                                                          double* __restrict__ out, long nout) {
   const long c = blockIdx.x;
   const int col = blockIdx.y * 64 + threadIdx.x;
   const long j = blockIdx.z;
   if (col >= width) return;
-  const double* src = in + j * nin * width;
-  double v[kFan];
-#pragma unroll
-  for (int i = 0; i < kFan; ++i) {
-    const long row = c * kFan + i;
-    v[i] = row < nin ? src[row * width + col] : 0.0;
-  }
-#pragma unroll
-  for (int h = kFan / 2; h > 0; h >>= 1)
-#pragma unroll
-    for (int i = 0; i < h; ++i) v[i] += v[i + h];
-  out[(j * nout + c) * width + col] = v[0];
+  out[(j * nout + c) * width + col] = column_sum(in + j * nin * width, nin, width, c, col);
 }
 
 // extra[j][b][i] = s_i sum_{k in chunk b} Qt[k][i] s_k for the kKch-wide
 // chunks b of k, and extra[j][nkb][i] = -w_i s_i V_i / N: summed over b and i,
-// s (Q s) - w s V / N, with (s, V) the field's column sums (the last
-// reduction pass left one row of 2 no values) and Qt = (diag(w) M)^T, M the
-// FP64 map s -> r-mean of vexc.  One thread per (i, chunk b, field j), all
-// kKch loads of a thread in flight together.
+// s (Q s) - w s V / N, with (s, V) the field's column sums and Qt =
+// (diag(w) M)^T, M the FP64 map s -> r-mean of vexc.  One thread per (i, chunk
+// b, field j), all kKch loads of a thread in flight together.  A block makes the
+// column sums it needs of the last nin <= kFan rows itself: a pass of its own
+// for them cost a launch, 6 us, in every evaluation, and 16 blocks re-reading
+// the rows from L2 cost less.
 constexpr int kKch = 24;
-__global__ __launch_bounds__(64) void mean_gemv_kernel(const double* __restrict__ sv, const double* __restrict__ qt,
-                                                       const double* __restrict__ w, int no, int nkb, double invN,
-                                                       double* __restrict__ extra) {
+__global__ __launch_bounds__(64) void mean_gemv_kernel(const double* __restrict__ in, int nin,
+                                                       const double* __restrict__ qt, const double* __restrict__ w,
+                                                       int no, int nkb, double invN, double* __restrict__ extra) {
   const int i = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y, j = blockIdx.z;
-  if (i >= no) return;
-  const double* s = sv + static_cast<long>(j) * 2 * no;
+  const int ic = min(i, no - 1);
+  const double* rows = in + static_cast<long>(j) * nin * (2 * no);
   double* out = extra + static_cast<long>(j) * (nkb + 1) * no;
-  const double si = s[i];
   if (b == nkb) {
-    out[static_cast<long>(nkb) * no + i] = -w[i] * si * s[no + i] * invN;
+    const double si = column_sum(rows, nin, 2 * no, 0, ic), vi = column_sum(rows, nin, 2 * no, 0, no + ic);
+    if (i < no) out[static_cast<long>(nkb) * no + i] = -w[i] * si * vi * invN;
     return;
   }
   double v[kKch];
 #pragma unroll
-  for (int q = 0; q < kKch; ++q) {
-    const int k = b * kKch + q;
-    v[q] = k < no ? qt[static_cast<long>(k) * no + i] * s[k] : 0.0;
-  }
+  for (int q = 0; q < kKch; ++q) v[q] = qt[static_cast<long>(min(b * kKch + q, no - 1)) * no + ic];
+  __shared__ double sk[kKch];
+  if (threadIdx.x < kKch)
+    sk[threadIdx.x] = column_sum(rows, nin, 2 * no, 0, min(b * kKch + static_cast<int>(threadIdx.x), no - 1));
+  const double si = column_sum(rows, nin, 2 * no, 0, ic);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kKch; ++q) v[q] = b * kKch + q < no ? v[q] * sk[q] : 0.0;
 #pragma unroll
   for (int h = 16; h > 0; h >>= 1)
 #pragma unroll
     for (int q = 0; q < h; ++q)
       if (q + h < kKch) v[q] += v[q + h];
-  out[static_cast<long>(b) * no + i] = si * v[0];
+  if (i < no) out[static_cast<long>(b) * no + i] = si * v[0];
 }
 
 long row_blocks_per_field(long N, int nb) { return nb == 1 ? (N + 63) / 64 : N / 64; }
@@ -197,7 +206,7 @@ void MeanModeFp64::run(const double* colpart, long N, int nb, double* work, doub
   double* buf[2] = {work, work + static_cast<size_t>(first) * nb * width};
   const double* in = colpart;
   int k = 0;
-  do {  // reduction passes down to one row of column sums per field
+  while (n > kFan) {  // reduction passes down to kFan rows of column sums per field
     const long m = chunks_after(n);
     hipLaunchKernelGGL(mean_colsum_kernel, dim3(static_cast<unsigned>(m), (width + 63) / 64, nb), dim3(64), 0, s,
                        in, n, width, buf[k], m);
@@ -205,10 +214,10 @@ void MeanModeFp64::run(const double* colpart, long N, int nb, double* work, doub
     in = buf[k];
     k ^= 1;
     n = m;
-  } while (n > 1);
+  }
   const int nkb = (no_ + kKch - 1) / kKch;
-  hipLaunchKernelGGL(mean_gemv_kernel, dim3((no_ + 63) / 64, nkb + 1, nb), dim3(64), 0, s, in, qt_, w_, no_, nkb,
-                     1.0 / static_cast<double>(N), extra);
+  hipLaunchKernelGGL(mean_gemv_kernel, dim3((no_ + 63) / 64, nkb + 1, nb), dim3(64), 0, s, in,
+                     static_cast<int>(n), qt_, w_, no_, nkb, 1.0 / static_cast<double>(N), extra);
   MDFT_HIP_CHECK(hipGetLastError());
 }
 
