@@ -371,9 +371,12 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
   using A = AngSizes<MMAX, MRSO>;
   constexpr int NP = A::np();
   // FP64 outputs are staged half the phi values at a time (the full stage of
-  // 64 x nphi npsi doubles would hold a CU to five blocks)
-  constexpr int kChunks = sizeof(TC) == 8 ? 2 : 1;
+  // 64 x nphi npsi doubles would hold a CU to five blocks), and so are rows of
+  // more than 64 values (mmax 6), of which the column sums below take one per
+  // lane
+  constexpr int kChunks = sizeof(TC) == 8 || A::kNjk > kWaveRows ? 2 : 1;
   constexpr int kJc = (A::kNphi + kChunks - 1) / kChunks;
+  static_assert(kJc * A::kNpsi <= 64, "one column per lane");
   __shared__ TC stage[kWaveRows * kJc * A::kNpsi];
   const int lane = threadIdx.x;
   const int q = blockIdx.x / kXcds;
