@@ -14,19 +14,6 @@ namespace {
 // 20.6, mmax 3 7.9 / 9.9).
 constexpr long kMinPoints = 120 * 64;
 
-// f(integral_constant<int, w>) for the wave-uniform w < N
-template <int N, int W = 0, typename F>
-__device__ __forceinline__ void dispatch_wave(int w, F&& f) {
-  if constexpr (W + 1 == N) {
-    f(std::integral_constant<int, W>{});
-  } else {
-    if (w == W)
-      f(std::integral_constant<int, W>{});
-    else
-      dispatch_wave<N, W + 1>(w, f);
-  }
-}
-
 // A block takes 64 consecutive r, one per lane, and its waves share out the
 // projections.  For each theta the 64 rows of (phi, psi) values go through LDS
 // (read in runs of nphi npsi, which is odd, so that a lane reads its own row

@@ -884,10 +884,16 @@ long proj2angl_row_blocks(long N) { return wave_row_blocks(N); }
 
 template <typename TP, typename TO, typename TC>
 void proj2angl_factorized(const ProjTables& t, long N, const cplx<TP>* p, TO* o, const TO* xi, TO* df,
-                          double rho0, double* partials, hipStream_t s, double* colpart, bool compact) {
+                          double rho0, double* partials, hipStream_t s, double* colpart, bool compact,
+                          bool mu_waves) {
   if (N == 0) return;
   const long nwb = wave_blocks(t, N);
   throw_if(nwb > 0x7fffffffL, "grid too large");
+  // the kernel here keeps the order of the mixed forms' sums
+  if constexpr (std::is_same<TO, TC>::value && std::is_same<TO, TP>::value)
+    if (mu_waves &&
+        launch_p2a_wave<TP, TO, TC>(t, N, p, o, xi, df, tabs_of<TC>(t, false), rho0, partials, s, colpart, compact))
+      return;
   const bool compiled = dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
     constexpr int MM = decltype(mm)::value, MR = decltype(mr)::value;
     if (compact)
@@ -960,13 +966,13 @@ template void angl2proj_factorized<double, float, float>(const ProjTables&, long
                                                          const double*, hipStream_t, bool, long);
 template void proj2angl_factorized<double, double, double>(const ProjTables&, long, const cplx<double>*, double*,
                                                            const double*, double*, double, double*, hipStream_t,
-                                                           double*, bool);
+                                                           double*, bool, bool);
 template void proj2angl_factorized<float, float, float>(const ProjTables&, long, const cplx<float>*, float*,
                                                         const float*, float*, double, double*, hipStream_t,
-                                                        double*, bool);
+                                                        double*, bool, bool);
 template void proj2angl_factorized<float, double, float>(const ProjTables&, long, const cplx<float>*, double*,
                                                          const double*, double*, double, double*, hipStream_t,
-                                                         double*, bool);
+                                                         double*, bool, bool);
 template void delta_rho<double>(const double*, double*, size_t, double, hipStream_t);
 template void delta_rho<float>(const float*, float*, size_t, double, hipStream_t);
 template int delta_f<double>(const double*, const double*, const double*, double*, long, int, double, double*, int,

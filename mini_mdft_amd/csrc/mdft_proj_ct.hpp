@@ -1,5 +1,5 @@
 // What the kernels for compile-time angular grids share (mdft_proj.hip,
-// mdft_a2p_wave.hip).
+// mdft_a2p_wave.hip, mdft_p2a_wave.hip).
 #pragma once
 
 #include <type_traits>
@@ -48,10 +48,29 @@ bool dispatch_angular(int mmax, int mrso, F&& f) {
   }
 }
 
+// f(integral_constant<int, w>) for the wave-uniform w < N
+template <int N, int W = 0, typename F>
+__device__ __forceinline__ void dispatch_wave(int w, F&& f) {
+  if constexpr (W + 1 == N) {
+    f(std::integral_constant<int, W>{});
+  } else {
+    if (w == W)
+      f(std::integral_constant<int, W>{});
+    else
+      dispatch_wave<N, W + 1>(w, f);
+  }
+}
+
 // angl2proj with one point per lane (mdft_a2p_wave.hip); false if the grid or
 // the number of points of a field is not one it serves
 template <typename TI, typename TP, typename TC>
 bool launch_a2p_wave(const ProjTables& t, long N, long field, const TI* o, cplx<TP>* p, const TabPtrs<TC>& tb,
                      const double* drho_rho0, hipStream_t s, bool compact);
+
+// proj2angl with a wave per mu2 (mdft_p2a_wave.hip); false if the grid is not one
+// it serves
+template <typename TP, typename TO, typename TC>
+bool launch_p2a_wave(const ProjTables& t, long N, const cplx<TP>* p, TO* o, const TO* xi, TO* df,
+                     const TabPtrs<TC>& tb, double rho0, double* partials, hipStream_t s, double* colpart, bool compact);
 
 }  // namespace mdft
