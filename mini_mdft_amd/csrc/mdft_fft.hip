@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_kernel(cplx<T>* __res
 }
 
 // one fused z/y pass over `planes` planes: the compile-time kernel for square
-// planes of the compile-time lengths up to 96 x 96, else fft_plane_kernel
+// planes of the compile-time lengths, else fft_plane_kernel
 template <typename T>
 void launch_plane(cplx<T>* data, const FftPlan1D& pz, const FftPlan1D& py, long planes, int threads, int sign,
                   hipStream_t s);
@@ -183,9 +183,9 @@ template <typename T>
 size_t plane_lds(int ny, int nz) {
   return (2 * static_cast<size_t>(ny) * (nz + 1) + ny + nz) * sizeof(cplx<T>);
 }
-// the fused z/y pass is used untuned when two planes fit in half of the
-// 160 KB LDS (at least two blocks of 8 waves per CU); the tuner also tries it
-// up to the whole LDS
+// the fused z/y pass is used untuned when its planes fit in half of the 160 KB
+// LDS (at least two blocks of 8 waves per CU); the tuner also tries it up to the
+// whole LDS
 constexpr size_t kPlaneLdsMax = 80 * 1024;
 
 // One block transforms a tile of W lines of length n.
@@ -367,13 +367,12 @@ const cplx<float>* FftPlan1D::twiddles<float>() const {
 
 Fft3dPlan::Fft3dPlan(int nx_, int ny_, int nz_) : nx(nx_), ny(ny_), nz(nz_), px(nx_), py(ny_), pz(nz_) {}
 
-bool Fft3dPlan::plane_ok(size_t elem, int threads) const {
-  (void)threads;
-  // the run-time plane kernel has radices up to 5; square planes of the
-  // compiled lengths have their own
-  return ny > 1 && nz > 1 && ((small_radices(py.st) && small_radices(pz.st)) || (ny == nz && plane_ct(ny, elem))) &&
+bool Fft3dPlan::plane_run_time(size_t elem) const {
+  return ny > 1 && nz > 1 && small_radices(py.st) && small_radices(pz.st) &&
          (2 * static_cast<size_t>(ny) * (nz + 1) + ny + nz) * elem <= kLdsMax;
 }
+
+bool Fft3dPlan::plane_ok(size_t elem) const { return (ny == nz && plane_ct(ny, elem)) || plane_run_time(elem); }
 
 template <typename T>
 void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, int sign, hipStream_t stream) const {
@@ -381,7 +380,7 @@ void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, in
   const long nxl = nx, nyl = ny, nzl = nz;
   const long planes = batch * nxl;
   if (c.plane) {
-    throw_if(!plane_ok(sizeof(cplx<T>), c.plane_threads) || planes > 0x7fffffffL ||
+    throw_if(!plane_ok(sizeof(cplx<T>)) || planes > 0x7fffffffL ||
                  (c.plane_threads != 256 && c.plane_threads != 512),
              "FFT: the fused plane pass does not apply to this shape");
     // z and y in one pass over each contiguous (y, z) plane
@@ -396,7 +395,9 @@ void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, in
 template <typename T>
 FftConfig Fft3dPlan::default_config() const {
   FftConfig c;
-  c.plane = plane_ok(sizeof(cplx<T>), 512) && plane_lds<T>(ny, nz) <= kPlaneLdsMax;
+  c.plane = plane_ok(sizeof(cplx<T>)) &&
+            (ny == nz && plane_ct(ny, sizeof(cplx<T>)) ? plane_ct_bytes(ny, sizeof(cplx<T>)) : plane_lds<T>(ny, nz)) <=
+                kPlaneLdsMax;
   c.plane_threads = 512;
   return c;
 }
@@ -476,7 +477,7 @@ FftConfig Fft3dPlan::autotune(long batch, hipStream_t s) const {
     axes.wx = x.first;
     best = axes;
     float best_t = z.second + y.second + x.second;
-    if (plane_ok(sizeof(cplx<T>), 512) && batch * nxl <= 0x7fffffffL) {
+    if (plane_ok(sizeof(cplx<T>)) && batch * nxl <= 0x7fffffffL) {
       for (int th : {256, 512}) {
         FftConfig c = axes;
         c.plane = true;

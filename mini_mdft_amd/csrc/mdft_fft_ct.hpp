@@ -13,6 +13,7 @@ namespace mdft {
 
 constexpr int kFftThreads = 256;
 constexpr int kMaxRadix = 13;
+constexpr size_t kLdsMax = 160 * 1024;
 
 template <typename T>
 __device__ __forceinline__ cplx<T> twiddle(const cplx<T>* tw, int t, int sign) {
@@ -192,39 +193,98 @@ __device__ __forceinline__ void ct_stockham_2d(cplx<T>* a, cplx<T>* b, const cpl
   }
 }
 
+// One stage of the lines of an LDS tile in place: every butterfly of the block in
+// registers between two barriers.
+template <typename T, int R, int N, int NS, int LS, int ES, int NLINES, int NTH, bool W_FAST>
+__device__ __forceinline__ void ct_stage_in_place(cplx<T>* buf, const cplx<T>* tw, int sign, int tid) {
+  constexpr int NB = N / R, TSTEP = N / (NS * R), TOTAL = NLINES * NB;
+  constexpr int ITERS = (TOTAL + NTH - 1) / NTH;
+  cplx<T> v[ITERS][R];
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i) {
+    const int beta = tid + i * NTH;
+    if (TOTAL % NTH == 0 || beta < TOTAL) {
+      const int w = W_FAST ? beta % NLINES : beta / NB, j = W_FAST ? beta / NLINES : beta % NB;
+      const int k = j % NS;
+      const cplx<T>* in = buf + w * LS + j * ES;
+      v[i][0] = in[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) v[i][r] = tw_mul<T>(in[r * NB * ES], twiddle<T>(tw, r * k * TSTEP, sign));
+      dft_fixed<T, R>(v[i], sign, tw, N);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i) {
+    const int beta = tid + i * NTH;
+    if (TOTAL % NTH == 0 || beta < TOTAL) {
+      const int w = W_FAST ? beta % NLINES : beta / NB, j = W_FAST ? beta / NLINES : beta % NB;
+      cplx<T>* out = buf + w * LS + ((j / NS) * NS * R + j % NS) * ES;
+#pragma unroll
+      for (int r = 0; r < R; ++r) out[r * NS * ES] = v[i][r];
+    }
+  }
+  __syncthreads();
+}
+
+template <typename T, int N, int LS, int ES, int NLINES, int NTH, bool W_FAST, int S = 0, int NS = 1>
+__device__ __forceinline__ void ct_stockham_in_place(cplx<T>* buf, const cplx<T>* tw, int sign, int tid) {
+  if constexpr (S < ct_nstages<N>()) {
+    constexpr int R = ct_radix<N>(S);
+    ct_stage_in_place<T, R, N, NS, LS, ES, NLINES, NTH, W_FAST>(buf, tw, sign, tid);
+    ct_stockham_in_place<T, N, LS, ES, NLINES, NTH, W_FAST, S + 1, NS * R>(buf, tw, sign, tid);
+  }
+}
+
+// The plane kernel's stages go back and forth between two padded planes while
+// three blocks of those fit on a CU (160 KB), else they work in place on one: a
+// block waits for its plane, transforms it, and stores it, and only another
+// block on the CU overlaps that.  One 3D transform of the stored channels, two
+// planes against one, microseconds: FP32 96^3 (one block a CU against two) 581
+// -> 454, 80^3 332 -> 261, 72^3 266 -> 198, 64^3 115 -> 108, FP64 64^3 263 -> 205,
+// 80^3 (two axis passes, as two planes do not fit) 662 -> 581.  With three blocks
+// and more the extra barrier of a stage is paid for at some lengths only: FP32
+// 4 x 48^3 185 -> 175, but 56^3 65 -> 68, 40^3 43 -> 45.
+constexpr bool plane_in_place(int n, size_t elem) {
+  return (2 * static_cast<size_t>(n) * (n + 1) + n) * elem > kLdsMax / 3;
+}
+// LDS of the kernel: one or two padded planes and the twiddles
+constexpr size_t plane_ct_bytes(int n, size_t elem) {
+  return ((plane_in_place(n, elem) ? 1 : 2) * static_cast<size_t>(n) * (n + 1) + n) * elem;
+}
+
 // fft_plane_kernel for an N x N plane with NTH threads
 template <typename T, int N, int NTH>
-__global__ __launch_bounds__(NTH) void fft_plane_ct_kernel(cplx<T>* __restrict__ data, const cplx<T>* __restrict__ twz_g,
-                                                           const cplx<T>* __restrict__ twy_g, int sign) {
+__global__ __launch_bounds__(NTH) void fft_plane_ct_kernel(cplx<T>* __restrict__ data, const cplx<T>* __restrict__ tw_g,
+                                                           int sign) {
   extern __shared__ unsigned char lds_raw[];
   constexpr int LD = N + 1, NN = N * N, ITERS = (NN + NTH - 1) / NTH;
-  cplx<T>* bufA = reinterpret_cast<cplx<T>*>(lds_raw);
-  cplx<T>* bufB = bufA + N * LD;
-  cplx<T>* twz = bufB + N * LD;
-  cplx<T>* twy = twz + N;
+  constexpr bool kInPlace = plane_in_place(N, sizeof(cplx<T>));
+  cplx<T>* buf = reinterpret_cast<cplx<T>*>(lds_raw);
+  cplx<T>* tw = buf + (kInPlace ? 1 : 2) * N * LD;
   const int tid = threadIdx.x;
-  if (tid < N) {
-    twz[tid] = twz_g[tid];
-    twy[tid] = twy_g[tid];
-  }
+  if (tid < N) tw[tid] = tw_g[tid];
   cplx<T>* plane = data + static_cast<long>(blockIdx.x) * NN;
 #pragma unroll
   for (int i = 0; i < ITERS; ++i) {
     const int t = tid + i * NTH;
-    if (NN % NTH == 0 || t < NN) bufA[(t / N) * LD + t % N] = plane[t];
+    if (NN % NTH == 0 || t < NN) buf[(t / N) * LD + t % N] = plane[t];
   }
   __syncthreads();
   // z along the rows, then y along the columns
-  ct_stockham_2d<T, N, LD, 1, N, NTH, false>(bufA, bufB, twz, sign, tid);
-  constexpr bool z_in_a = ct_nstages<N>() % 2 == 0;
-  cplx<T>* a = z_in_a ? bufA : bufB;
-  cplx<T>* b = z_in_a ? bufB : bufA;
-  ct_stockham_2d<T, N, 1, LD, N, NTH, true>(a, b, twy, sign, tid);
-  const cplx<T>* res = bufA;  // two axes of the same stage count end where they began
+  if constexpr (kInPlace) {
+    ct_stockham_in_place<T, N, LD, 1, N, NTH, false>(buf, tw, sign, tid);
+    ct_stockham_in_place<T, N, 1, LD, N, NTH, true>(buf, tw, sign, tid);
+  } else {  // two axes of the same stage count end where they began
+    cplx<T>* second = buf + N * LD;
+    constexpr bool odd = ct_nstages<N>() % 2 == 1;
+    ct_stockham_2d<T, N, LD, 1, N, NTH, false>(buf, second, tw, sign, tid);
+    ct_stockham_2d<T, N, 1, LD, N, NTH, true>(odd ? second : buf, odd ? buf : second, tw, sign, tid);
+  }
 #pragma unroll
   for (int i = 0; i < ITERS; ++i) {
     const int t = tid + i * NTH;
-    if (NN % NTH == 0 || t < NN) plane[t] = res[(t / N) * LD + t % N];
+    if (NN % NTH == 0 || t < NN) plane[t] = buf[(t / N) * LD + t % N];
   }
 }
 
@@ -289,17 +349,14 @@ template <typename T>
 constexpr size_t axis_lds(int n, int W) {
   return (2 * static_cast<size_t>(W) * (n + 1) + n) * sizeof(cplx<T>);
 }
-constexpr size_t kLdsMax = 160 * 1024;
 
 // launches the compile-time axis kernel of (n, W), if there is one
 template <typename T>
 bool launch_axis_ct(cplx<T>* data, const cplx<T>* tw, int n, int W, bool strided, int sign, long nlines_or_outer,
                     long S, hipStream_t stream);
-// whether n x n planes of elem-byte values have a compile-time kernel: two
-// padded planes and the twiddles in LDS (n up to 99 in FP32, 70 in FP64)
-inline bool plane_ct(int n, size_t elem) {
-  return ct_length(n) && n <= 99 && (2 * static_cast<size_t>(n) * (n + 1) + 2 * n) * elem <= kLdsMax;
-}
+// whether n x n planes of elem-byte values have a compile-time kernel (n up to
+// 128 in FP32, 100 in FP64)
+inline bool plane_ct(int n, size_t elem) { return ct_length(n) && plane_ct_bytes(n, elem) <= kLdsMax; }
 // launches it, if there is one (the lengths that have one thread count take
 // that one, whatever threads says)
 template <typename T>

@@ -8,7 +8,7 @@ namespace {
 // plane_ct at compile time
 template <typename T, int N>
 constexpr bool plane_fits() {
-  return N >= 8 && N <= 99 && (2 * static_cast<size_t>(N) * (N + 1) + 2 * N) * sizeof(cplx<T>) <= kLdsMax;
+  return plane_ct_bytes(N, sizeof(cplx<T>)) <= kLdsMax;
 }
 // The lengths whose planes are compiled with 256 and with 512 threads (the
 // tuner's choice).  The others have one count: up to 32 a stage has at most 256
@@ -26,9 +26,9 @@ bool launch_plane_ct(cplx<T>* data, const cplx<T>* tw, int n, long planes, int t
   for_length(n, CtLengths{}, [&](auto nn) {
     constexpr int N = decltype(nn)::value;
     if constexpr (plane_fits<T, N>()) {
-      constexpr size_t lds = (2 * static_cast<size_t>(N) * (N + 1) + 2 * N) * sizeof(cplx<T>);
+      constexpr size_t lds = plane_ct_bytes(N, sizeof(cplx<T>));
       auto go = [&](auto kernel, int th) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(planes)), dim3(th), lds, s, data, tw, tw, sign);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(planes)), dim3(th), lds, s, data, tw, sign);
         MDFT_HIP_CHECK(hipGetLastError());
         done = true;
       };
