@@ -25,8 +25,8 @@ constexpr long kMinPoints = 120 * 64;
 // its projections.  A fifth of the products of one thread per (r, theta, mup,
 // mu2) with its operands in LDS, which that kernel spent its time reading:
 // 64^3 mmax 5 FP64 483 -> 247 us (1.0 GB, 207 us at the copy rate), FP32 291 ->
-// 126 (104 us); 45x36x50 mmax 4 FP32 54 -> 30.  At most 13 sums per wave (six
-// waves at mmax 5): 26 sums 315 us in FP64 (256 registers, one wave per SIMD),
+// 126 (104 us); 45x36x50 mmax 4 FP32 54 -> 30.  At most 13 sums per wave
+// (seven waves at mmax 5): 26 sums 315 us in FP64 (256 registers, one wave per SIMD),
 // 21 277, 16 284, 10 284, in FP32 123, 147, 146, 133.  Each role is a whole copy
 // of the loop: with the roles inside one loop the compiler kept part of the sums
 // in memory (659 us).

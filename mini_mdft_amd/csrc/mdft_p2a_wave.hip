@@ -114,7 +114,7 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
     double* __restrict__ colpart) {
   using Z = A2pSizes<MMAX, MRSO, 1>;
   constexpr int NPHI = Z::kNphi, NPSI = Z::kNpsi, NMU2 = Z::kNmu2, NJK = NPHI * NPSI, NO = Z::kNo, NTH = Z::kNth;
-  constexpr int kG = 64 * NMU2 / NJK, kSteps = (kRows + kG - 1) / kG;  // rows of one step of the block, steps
+  constexpr int kG = 64 * NMU2 / NJK < 16 ? 64 * NMU2 / NJK : 16, kSteps = (kRows + kG - 1) / kG;  // rows of one step of the block, steps
   __shared__ alignas(8) TC stage[kRows * NJK];
   __shared__ double red[NMU2];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -241,19 +241,17 @@ bool launch_p2a_wave(const ProjTables& t, long N, const cplx<TP>* p, TO* o, cons
   bool done = false;
   dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
     constexpr int MMAX = decltype(mm)::value, MRSO = decltype(mr)::value;
-    if constexpr (MMAX / MRSO >= 1) {
-      const long nrb = (N + kRows - 1) / kRows, blocks = (nrb + kXcds - 1) / kXcds * kXcds * t.ntheta;
-      auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * (MMAX / MRSO + 1)), 0, s, p, o, xi,
-                           df, t.w, N, nrb, tb, rho0, partials, colpart);
-        MDFT_HIP_CHECK(hipGetLastError());
-        done = true;
-      };
-      if (compact)
-        go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, true>);
-      else
-        go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, false>);
-    }
+    const long nrb = (N + kRows - 1) / kRows, blocks = (nrb + kXcds - 1) / kXcds * kXcds * t.ntheta;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * (MMAX / MRSO + 1)), 0, s, p, o, xi,
+                         df, t.w, N, nrb, tb, rho0, partials, colpart);
+      MDFT_HIP_CHECK(hipGetLastError());
+      done = true;
+    };
+    if (compact)
+      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, true>);
+    else
+      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, false>);
   });
   return done;
 }

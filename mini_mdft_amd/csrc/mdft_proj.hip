@@ -337,7 +337,8 @@ __global__ __launch_bounds__(kThreads) void proj2angl_kernel(const cplx<TP>* __r
   if (xi != nullptr) block_sum_store<TC>(acc_ff, partials + blockIdx.x);
 }
 
-// proj2angl for angular grids with compile-time sizes: one 64-lane block per
+// proj2angl of the mixed forms for angular grids with compile-time sizes (the
+// FP64 and FP32 forms: mdft_p2a_wave.hip): one 64-lane block per
 // (64 consecutive r, theta).  Each lane keeps its S[mup][mu2] in registers
 // (the m sums in the same ascending-m order as proj2angl_kernel), runs the
 // phi sums on the (mup, -mup) pairs, Z = S_0 + sum_{mup > 0} (A cos + i B sin)
@@ -370,11 +371,9 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
                                                             double* __restrict__ colpart) {
   using A = AngSizes<MMAX, MRSO>;
   constexpr int NP = A::np();
-  // FP64 outputs are staged half the phi values at a time (the full stage of
-  // 64 x nphi npsi doubles would hold a CU to five blocks), and so are rows of
-  // more than 64 values (mmax 6), of which the column sums below take one per
-  // lane
-  constexpr int kChunks = sizeof(TC) == 8 || A::kNjk > kWaveRows ? 2 : 1;
+  // rows of more than 64 values (mmax 6) are staged half the phi values at a
+  // time: the column sums below take one per lane
+  constexpr int kChunks = A::kNjk > kWaveRows ? 2 : 1;
   constexpr int kJc = (A::kNphi + kChunks - 1) / kChunks;
   static_assert(kJc * A::kNpsi <= 64, "one column per lane");
   __shared__ TC stage[kWaveRows * kJc * A::kNpsi];
@@ -468,9 +467,8 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
       // get_delta_f with the column sums: lane jk owns orientation th * nphi
       // npsi + c0 + jk and walks the block's rows, so that its sums over r of
       // xi^2 - 1 and of vexc build up in registers (each row's W values are
-      // one contiguous run of xi and df; for the mixed forms this walk also
-      // measured faster than the row-major one below, 0.358 against 0.371 ms
-      // at 64^3, and in FP64 the same, 1.11 against 1.10 ms)
+      // one contiguous run of xi and df; this walk also measured faster than
+      // the row-major one below, 0.358 against 0.371 ms at 64^3)
       constexpr int kRB = 32;  // rows per batch of loads in flight
       const int nrow = static_cast<int>(min(static_cast<long>(kWaveRows), N - r0));
       const bool on = lane < W;
@@ -508,8 +506,8 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
       // in flight before the arithmetic.  The mixed forms (FP32 arithmetic,
       // FP64 fields) take all kE at once: at mmax 5 that waits out one HBM
       // latency instead of five and measured 3% faster, at the same three
-      // waves per SIMD.  The FP64 and FP32 forms keep batches of 11 (one
-      // batch would nearly double their registers at mmax 5).
+      // waves per SIMD.  FP32 fields keep batches of 11 (one batch would
+      // nearly double their registers at mmax 5).
       constexpr bool kMixed = std::is_same<TC, float>::value && std::is_same<TO, double>::value;
       constexpr int kB = kMixed && kE <= 64 ? kE : 11;
       for (int i0 = 0; i0 < kE; i0 += kB) {
@@ -890,21 +888,22 @@ void proj2angl_factorized(const ProjTables& t, long N, const cplx<TP>* p, TO* o,
   const long nwb = wave_blocks(t, N);
   throw_if(nwb > 0x7fffffffL, "grid too large");
   // the kernel here keeps the order of the mixed forms' sums
+  bool compiled = false;
   if constexpr (std::is_same<TO, TC>::value && std::is_same<TO, TP>::value)
-    if (mu_waves &&
-        launch_p2a_wave<TP, TO, TC>(t, N, p, o, xi, df, tabs_of<TC>(t, false), rho0, partials, s, colpart, compact))
-      return;
-  const bool compiled = dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
-    constexpr int MM = decltype(mm)::value, MR = decltype(mr)::value;
-    if (compact)
-      hipLaunchKernelGGL((proj2angl_wave_kernel<MM, MR, TP, TO, TC, true>), dim3(static_cast<unsigned>(nwb)),
-                         dim3(64), 0, s, p, o, xi, df, t.w, N, wave_row_blocks(N), tabs_of<TC>(t, false), rho0,
-                         partials, colpart);
-    else
-      hipLaunchKernelGGL((proj2angl_wave_kernel<MM, MR, TP, TO, TC, false>), dim3(static_cast<unsigned>(nwb)),
-                         dim3(64), 0, s, p, o, xi, df, t.w, N, wave_row_blocks(N), tabs_of<TC>(t, false), rho0,
-                         partials, colpart);
-  });
+    compiled = mu_waves &&
+               launch_p2a_wave<TP, TO, TC>(t, N, p, o, xi, df, tabs_of<TC>(t, false), rho0, partials, s, colpart, compact);
+  if constexpr (!std::is_same<TC, double>::value)
+    compiled = compiled || dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
+      constexpr int MM = decltype(mm)::value, MR = decltype(mr)::value;
+      const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nwb)), dim3(64), 0, s, p, o, xi, df, t.w, N,
+                           wave_row_blocks(N), tabs_of<TC>(t, false), rho0, partials, colpart);
+      };
+      if (compact)
+        go(proj2angl_wave_kernel<MM, MR, TP, TO, TC, true>);
+      else
+        go(proj2angl_wave_kernel<MM, MR, TP, TO, TC, false>);
+    });
   if (compiled) {
     MDFT_HIP_CHECK(hipGetLastError());
     return;

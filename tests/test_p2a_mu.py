@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-GRIDS = [(1, 1), (2, 1), (2, 2), (3, 1), (3, 2), (4, 2), (5, 2), (6, 2)]
+GRIDS = [(1, 1), (1, 2), (2, 1), (2, 2), (3, 1), (3, 2), (4, 2), (5, 2), (6, 2)]
 
 
 @pytest.mark.parametrize("mmax,mrso", GRIDS)
