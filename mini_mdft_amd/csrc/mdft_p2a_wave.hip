@@ -2,6 +2,7 @@
 // block of one wave per mu2 for each (64 consecutive r, theta) (see
 // mdft_proj.hip for the sums).
 #include "mdft_proj_ct.hpp"
+#include "mdft_rows.hpp"
 
 namespace mdft {
 
@@ -114,7 +115,8 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
     double* __restrict__ colpart) {
   using Z = A2pSizes<MMAX, MRSO, 1>;
   constexpr int NPHI = Z::kNphi, NPSI = Z::kNpsi, NMU2 = Z::kNmu2, NJK = NPHI * NPSI, NO = Z::kNo, NTH = Z::kNth;
-  constexpr int kG = 64 * NMU2 / NJK < 16 ? 64 * NMU2 / NJK : 16, kSteps = (kRows + kG - 1) / kG;  // rows of one step of the block, steps
+  using Walk = RowWalk<NJK, 64 * NMU2, kRows>;
+  constexpr int kG = Walk::kG, kSteps = Walk::kSteps;
   __shared__ alignas(8) TC stage[kRows * NJK];
   __shared__ double red[NMU2];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -130,10 +132,9 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
   // of a step is a scalar plus a constant of the thread
   const int sub = tid / NJK, col = tid - sub * NJK;
   const bool on = sub < kG;
-  // byte offset of the thread's value in step u; a step past the last row
-  // repeats the thread's last one
-  const unsigned off0 = on ? (sub * NO + col) * sizeof(TO) : 0;
-  const int reach = on ? max(last - sub, 0) / kG : 0;
+  // byte offset of the thread's value in step u (Walk::row(sub, u, last))
+  const unsigned off0 = on ? (Walk::first(sub, last) * NO + col) * sizeof(TO) : 0;
+  const int reach = on ? Walk::reach(sub, last) : 0;
   const auto off = [&](int u) { return off0 + min(u, reach) * static_cast<unsigned>(kG * NO * sizeof(TO)); };
   TO x[kSteps];
   const auto request = [&] {
