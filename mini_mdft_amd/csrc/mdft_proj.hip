@@ -371,12 +371,8 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
                                                             double* __restrict__ colpart) {
   using A = AngSizes<MMAX, MRSO>;
   constexpr int NP = A::np();
-  // rows of more than 64 values (mmax 6) are staged half the phi values at a
-  // time: the column sums below take one per lane
-  constexpr int kChunks = A::kNjk > kWaveRows ? 2 : 1;
-  constexpr int kJc = (A::kNphi + kChunks - 1) / kChunks;
-  static_assert(kJc * A::kNpsi <= 64, "one column per lane");
-  __shared__ TC stage[kWaveRows * kJc * A::kNpsi];
+  constexpr int W = A::kNjk;  // outputs of a row
+  __shared__ TC stage[kWaveRows * W];
   const int lane = threadIdx.x;
   const int q = blockIdx.x / kXcds;
   const int th = q % A::kNth;
@@ -426,17 +422,14 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
   }
   double acc_ff = 0.0;
   const long base = r0 * A::kNo + th * A::kNjk;
-  // the (phi, psi) outputs of chunk c: phi in [c kJc, c kJc + jn), their nphi
-  // npsi columns [c0, c0 + W) of the row's run, staged as [64 rows][W]
-  const auto chunk = [&](auto cc) {
-    constexpr int c = decltype(cc)::value;
-    constexpr int j0 = c * kJc, jn = A::kNphi - j0 < kJc ? A::kNphi - j0 : kJc;
-    constexpr int W = jn * A::kNpsi, c0 = j0 * A::kNpsi;
-    if (c > 0) __syncthreads();  // the previous chunk's epilogue has read the stage
+  // The phi and psi sums and the epilogue.  A generic lambda, whose loops unroll
+  // before it is inlined: written into the kernel itself they left 127 registers
+  // at mmax 6 and few projections in flight (X6F, 64^3: 1443 us against 752).
+  const auto outputs = [&](auto first) {
+    constexpr int j0 = decltype(first)::value;
     TC* out = stage + lane * W;
 #pragma unroll
-    for (int jj = 0; jj < jn; ++jj) {
-      const int j = j0 + jj;
+    for (int j = j0; j < A::kNphi; ++j) {
       TC zr[A::kNmu2], zi[A::kNmu2];
 #pragma unroll
       for (int b = 0; b < A::kNmu2; ++b) {
@@ -457,7 +450,7 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
           const cplx<TC> e = tb.epsi[b * A::kNpsi + k];
           v += static_cast<TC>(2) * (zr[b] * e.x - zi[b] * e.y);
         }
-        out[jj * A::kNpsi + k] = v;
+        out[j * A::kNpsi + k] = v;
       }
     }
     __syncthreads();
@@ -465,41 +458,47 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
     constexpr int kE = W;  // elements per lane (64 rows x W columns)
     if (colpart != nullptr && xi != nullptr) {
       // get_delta_f with the column sums: lane jk owns orientation th * nphi
-      // npsi + c0 + jk and walks the block's rows, so that its sums over r of
+      // npsi + jk and walks the block's rows, so that its sums over r of
       // xi^2 - 1 and of vexc build up in registers (each row's W values are
       // one contiguous run of xi and df; this walk also measured faster than
-      // the row-major one below, 0.358 against 0.371 ms at 64^3)
+      // the row-major one below, 0.358 against 0.371 ms at 64^3).  A row of
+      // mmax 6 has 91 values: a second walk takes the columns from 64 on (staged
+      // and walked in two halves instead, the sums and both walks took 340
+      // registers: X6F, 64^3, 1075 us against 752)
       constexpr int kRB = 32;  // rows per batch of loads in flight
       const int nrow = static_cast<int>(min(static_cast<long>(kWaveRows), N - r0));
-      const bool on = lane < W;
-      const int jk = on ? lane : 0;
-      double cs = 0.0, cv = 0.0;
-      for (int rl0 = 0; rl0 < kWaveRows; rl0 += kRB) {
-        double xv[kRB];
 #pragma unroll
-        for (int b = 0; b < kRB; ++b) {
-          const int rl = min(rl0 + b, nrow - 1);
-          xv[b] = static_cast<double>(xi[base + static_cast<long>(rl) * A::kNo + c0 + jk]);
-        }
+      for (int w0 = 0; w0 < W; w0 += 64) {
+        const bool on = W - w0 >= 64 || w0 + lane < W;
+        const int jk = W - w0 >= 64 ? w0 + lane : min(w0 + lane, W - 1);
+        double cs = 0.0, cv = 0.0;
+        for (int rl0 = 0; rl0 < kWaveRows; rl0 += kRB) {
+          double xv[kRB];
 #pragma unroll
-        for (int b = 0; b < kRB; ++b) {
-          const int rl = rl0 + b;
-          if (on && rl < nrow) {
-            const double x = xv[b];
-            const double vx = static_cast<double>(static_cast<TO>(stage[rl * W + jk]));
-            const double x2m1 = x * x - 1.0;
-            acc_ff += vx * wth * x2m1;
-            df[base + static_cast<long>(rl) * A::kNo + c0 + jk] = static_cast<TO>(2.0 * rho0 * x * vx);
-            cs += x2m1;
-            cv += vx;
+          for (int b = 0; b < kRB; ++b) {
+            const int rl = min(rl0 + b, nrow - 1);
+            xv[b] = static_cast<double>(xi[base + static_cast<long>(rl) * A::kNo + jk]);
+          }
+#pragma unroll
+          for (int b = 0; b < kRB; ++b) {
+            const int rl = rl0 + b;
+            if (on && rl < nrow) {
+              const double x = xv[b];
+              const double vx = static_cast<double>(static_cast<TO>(stage[rl * W + jk]));
+              const double x2m1 = x * x - 1.0;
+              acc_ff += vx * wth * x2m1;
+              df[base + static_cast<long>(rl) * A::kNo + jk] = static_cast<TO>(2.0 * rho0 * x * vx);
+              cs += x2m1;
+              cv += vx;
+            }
           }
         }
-      }
-      if (on) {
-        // colpart[rb][0][io] = sum_r (xi^2 - 1), colpart[rb][1][io] = sum_r vexc
-        double* cp = colpart + rb * (2 * A::kNo) + th * A::kNjk + c0 + jk;
-        cp[0] = cs;
-        cp[A::kNo] = cv;
+        if (on) {
+          // colpart[rb][0][io] = sum_r (xi^2 - 1), colpart[rb][1][io] = sum_r vexc
+          double* cp = colpart + rb * (2 * A::kNo) + th * A::kNjk + jk;
+          cp[0] = cs;
+          cp[A::kNo] = cv;
+        }
       }
     } else if (xi != nullptr && r0 + kWaveRows <= N) {
       // full block: batches of kB elements per lane with all their xi loads
@@ -516,14 +515,14 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
         for (int b = 0; b < kB; ++b) {
           const int e = lane + 64 * min(i0 + b, kE - 1);
           const int rl = e / W, jk = e - rl * W;
-          xv[b] = static_cast<double>(xi[base + static_cast<long>(rl) * A::kNo + c0 + jk]);
+          xv[b] = static_cast<double>(xi[base + static_cast<long>(rl) * A::kNo + jk]);
         }
 #pragma unroll
         for (int b = 0; b < kB; ++b) {
           if (i0 + b < kE) {
             const int e = lane + 64 * (i0 + b);
             const int rl = e / W, jk = e - rl * W;
-            const long g = base + static_cast<long>(rl) * A::kNo + c0 + jk;
+            const long g = base + static_cast<long>(rl) * A::kNo + jk;
             const double x = xv[b];
             const double vx = static_cast<double>(static_cast<TO>(stage[e]));
             acc_ff += vx * wth * (x * x - 1.0);
@@ -536,7 +535,7 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
       for (int e = lane; e < kWaveRows * W; e += 64) {
         const int rl = e / W, jk = e - rl * W;
         if (r0 + rl < N) {
-          const long g = base + static_cast<long>(rl) * A::kNo + c0 + jk;
+          const long g = base + static_cast<long>(rl) * A::kNo + jk;
           const TC v = stage[e];
           if (xi == nullptr) {
             o[g] = static_cast<TO>(v);
@@ -550,8 +549,7 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
       }
     }
   };
-  chunk(std::integral_constant<int, 0>{});
-  if constexpr (kChunks > 1) chunk(std::integral_constant<int, 1>{});
+  outputs(std::integral_constant<int, 0>{});
   if (xi != nullptr) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) acc_ff += __shfl_xor(acc_ff, off);
