@@ -108,13 +108,22 @@ __device__ __forceinline__ void p2a_wave(const cplx<TP>* __restrict__ p, long N,
 // -> 207, 32^3 mmax 5 37 -> 31, 64^3 mmax 5 241 -> 252 (channels a power of two
 // apart; 63^3 244 -> 224, 80^3 461 -> 459).  With the xi requested first and 172
 // registers FP64 64^3 took 639, held to 168 and 128 registers 804 and 1150.
-template <int MMAX, int MRSO, typename TP, typename TO, typename TC, bool CP>
+//
+// FUSED: with get_delta_f, if that is known at compile time (FP64 in the full
+// order).  Elsewhere it is a branch on xi, behind which the request of xi stays
+// in front of the phi sums: FP64 64^3 mmax 5, compact order, 451 us, and 468 where
+// the compiler moves it behind them.  In the full order, whose mu2 = 0 has 36
+// projections for 21, the early request needs more than 256 registers and leaves
+// one wave per SIMD: 640 us against 530, and 506 against 388 for proj2angl alone,
+// which requests nothing (FP32 fits either way).
+template <int MMAX, int MRSO, typename TP, typename TO, typename TC, bool CP, bool FUSED>
 __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
     const cplx<TP>* __restrict__ p, TO* __restrict__ o, const TO* __restrict__ xi, TO* __restrict__ df,
     const double* __restrict__ wq, long N, long nrb, TabPtrs<TC> tb, double rho0, double* __restrict__ partials,
     double* __restrict__ colpart) {
   using Z = A2pSizes<MMAX, MRSO, 1>;
   constexpr int NPHI = Z::kNphi, NPSI = Z::kNpsi, NMU2 = Z::kNmu2, NJK = NPHI * NPSI, NO = Z::kNo, NTH = Z::kNth;
+  const bool fused = sizeof(TC) == 8 && !CP ? FUSED : xi != nullptr;
   using Walk = RowWalk<NJK, 64 * NMU2, kRows>;
   constexpr int kG = Walk::kG, kSteps = Walk::kSteps;
   __shared__ alignas(8) TC stage[kRows * NJK];
@@ -138,7 +147,7 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
   const auto off = [&](int u) { return off0 + min(u, reach) * static_cast<unsigned>(kG * NO * sizeof(TO)); };
   TO x[kSteps];
   const auto request = [&] {
-    if (xi == nullptr) return;
+    if (!fused) return;
     const char* from = reinterpret_cast<const char*>(xi + base);
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) x[u] = *reinterpret_cast<const TO*>(from + off(u));
@@ -175,10 +184,10 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
   }
   __syncthreads();
   double acc = 0.0, cs = 0.0, cv = 0.0;
-  char* to = reinterpret_cast<char*>((xi == nullptr ? o : df) + base);
+  char* to = reinterpret_cast<char*>((fused ? df : o) + base);
   const auto put = [&](int u) {
     const TO v = static_cast<TO>(stage[(u * kG + sub) * NJK + col]);
-    if (xi == nullptr) {
+    if (!fused) {
       *reinterpret_cast<TO*>(to + off(u)) = v;
     } else {
       const double xv = static_cast<double>(x[u]), vx = static_cast<double>(v);
@@ -200,7 +209,7 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
         if (sub <= last && u <= reach) put(u);
     }
   }
-  if (colpart != nullptr && xi != nullptr) {
+  if (colpart != nullptr && fused) {
     // colpart[rb][0][io] = sum_r (xi^2 - 1), colpart[rb][1][io] = sum_r vexc:
     // the threads' sums, then those of a column in the order of sub
     static_assert(2 * kG * sizeof(double) <= kRows * sizeof(TC), "the stage holds the sums");
@@ -222,7 +231,7 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
       cp[NO] = s1;
     }
   }
-  if (xi != nullptr) {
+  if (fused) {
 #pragma unroll
     for (int h = 32; h > 0; h >>= 1) acc += __shfl_xor(acc, h);
     if (lane == 0) red[wave] = acc;
@@ -250,9 +259,11 @@ bool launch_p2a_wave(const ProjTables& t, long N, const cplx<TP>* p, TO* o, cons
       done = true;
     };
     if (compact)
-      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, true>);
+      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, true, true>);
+    else if (sizeof(TC) == 4 || xi != nullptr)
+      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, false, true>);
     else
-      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, false>);
+      go(proj2angl_mu_kernel<MMAX, MRSO, TP, TO, TC, false, sizeof(TC) == 4>);
   });
   return done;
 }
