@@ -301,12 +301,12 @@ int mdft_proj2angl(mdft_opt_t h, const void* p, void* o, void* stream) {
       case MDFT_FP64:
         proj2angl_factorized<double, double, double>(*h->tab, h->N, static_cast<const cplx<double>*>(p),
                                                      static_cast<double*>(o), nullptr, nullptr, 0.0, nullptr, s, nullptr,
-                                                     false, true);
+                                                     false, proj2angl_mu_waves(*h->tab, true, h->N, false));
         break;
       case MDFT_FP32:
         proj2angl_factorized<float, float, float>(*h->tab, h->N, static_cast<const cplx<float>*>(p),
                                                   static_cast<float*>(o), nullptr, nullptr, 0.0, nullptr, s, nullptr, false,
-                                                  true);
+                                                  proj2angl_mu_waves(*h->tab, false, h->N, false));
         break;
       case MDFT_MIXED_X6F:
         h->gemm->proj2angl(h->N, static_cast<const cplx<float>*>(p), static_cast<float*>(o), nullptr, nullptr, 0.0,
@@ -641,7 +641,7 @@ static void energy_impl(mdft_solver_t h, int nb, const void* xi, void* df, doubl
       h->conv->dev->execute<double>(p, eps, s, tm, nb, h->compact);
       proj2angl_factorized<double, double, double>(*h->tab, Nb, p, nullptr, static_cast<const double*>(xi),
                                                    static_cast<double*>(df), rho0, h->partials, s, colp,
-                                                   h->compact, true);
+                                                   h->compact, proj2angl_mu_waves(*h->tab, true, h->N, true));
       break;
     }
     case MDFT_FP32: {
@@ -651,7 +651,7 @@ static void energy_impl(mdft_solver_t h, int nb, const void* xi, void* df, doubl
       h->conv->dev->execute<float>(p, eps, s, tm, nb, h->compact);
       proj2angl_factorized<float, float, float>(*h->tab, Nb, p, nullptr, static_cast<const float*>(xi),
                                                 static_cast<float*>(df), rho0, h->partials, s, colp,
-                                                h->compact, true);
+                                                h->compact, proj2angl_mu_waves(*h->tab, false, h->N, true));
       break;
     }
     case MDFT_MIXED_X6F: {

@@ -245,6 +245,17 @@ __global__ __launch_bounds__((64 * (MMAX / MRSO + 1))) void proj2angl_mu_kernel(
 
 }  // namespace
 
+bool proj2angl_mu_waves(const ProjTables& t, bool fp64, long field, bool fused) {
+  // Fused FP32 at mmax 5, single wave against these (us): 48^3 97 / 90, 64 x 64 x
+  // 32 (2^17) 115.7 / 117.4, 63 x 64^2 219 / 224, 64^3 237 / 250, 96 x 64^2 342 /
+  // 347, 80^3 450 / 452, 128 x 64^2 481 / 507: once the chip is full the single
+  // wave, which has every channel of its rows in flight, gains on channels that
+  // are a power of two apart and loses nowhere.  Alone (63 / 52 at 48^3, 217 /
+  // 212 at 64^3), at the other mmax (64^3: mmax 4 159 / 156, mmax 6 782 / 530) and
+  // in FP64 the wave per mu2 is as fast or faster.
+  return fp64 || !fused || t.mmax != 5 || t.mrso != 2 || field < (1L << 17);
+}
+
 template <typename TP, typename TO, typename TC>
 bool launch_p2a_wave(const ProjTables& t, long N, const cplx<TP>* p, TO* o, const TO* xi, TO* df,
                      const TabPtrs<TC>& tb, double rho0, double* partials, hipStream_t s, double* colpart, bool compact) {

@@ -337,8 +337,8 @@ __global__ __launch_bounds__(kThreads) void proj2angl_kernel(const cplx<TP>* __r
   if (xi != nullptr) block_sum_store<TC>(acc_ff, partials + blockIdx.x);
 }
 
-// proj2angl of the mixed forms for angular grids with compile-time sizes (the
-// FP64 and FP32 forms: mdft_p2a_wave.hip): one 64-lane block per
+// proj2angl of the mixed forms, and of FP32 where proj2angl_mu_waves leaves it, for
+// angular grids with compile-time sizes (else mdft_p2a_wave.hip): one 64-lane block per
 // (64 consecutive r, theta).  Each lane keeps its S[mup][mu2] in registers
 // (the m sums in the same ascending-m order as proj2angl_kernel), runs the
 // phi sums on the (mup, -mup) pairs, Z = S_0 + sum_{mup > 0} (A cos + i B sin)
@@ -885,7 +885,7 @@ void proj2angl_factorized(const ProjTables& t, long N, const cplx<TP>* p, TO* o,
   if (N == 0) return;
   const long nwb = wave_blocks(t, N);
   throw_if(nwb > 0x7fffffffL, "grid too large");
-  // the kernel here keeps the order of the mixed forms' sums
+  // the single-wave kernel keeps the order of the mixed forms' sums
   bool compiled = false;
   if constexpr (std::is_same<TO, TC>::value && std::is_same<TO, TP>::value)
     compiled = mu_waves &&

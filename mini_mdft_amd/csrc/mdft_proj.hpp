@@ -110,12 +110,15 @@ bool angl2proj_compiled(const ProjTables& t, bool fp64);
 // epilogue also writes, per block of 64 rows rb, the column sums over its
 // rows: colpart[rb][0][io] = sum_r (xi^2 - 1), colpart[rb][1][io] = sum_r vexc.
 // With compact, p holds the stored channels of the compact channel order
-// (compile-time grids only).  mu_waves: the FP64 and FP32 forms, which take the
-// faster kernel of mdft_p2a_wave.hip where it serves.
+// (compile-time grids only).  mu_waves: take the kernel of mdft_p2a_wave.hip
+// where it has the grid (FP64 and FP32 forms; proj2angl_mu_waves).
 template <typename TP, typename TO, typename TC>
 void proj2angl_factorized(const ProjTables& t, long N, const cplx<TP>* p, TO* o, const TO* xi, TO* df,
                           double rho0, double* partials, hipStream_t s, double* colpart = nullptr,
                           bool compact = false, bool mu_waves = false);
+// whether the wave per mu2 is the faster kernel for an FP64 (fp64) or FP32 form
+// with fields of so many points
+bool proj2angl_mu_waves(const ProjTables& t, bool fp64, long field, bool fused);
 // whether proj2angl_factorized can write column sums for this grid, and the
 // row blocks (64 rows each) it writes them for
 bool proj2angl_has_column_sums(const ProjTables& t);
