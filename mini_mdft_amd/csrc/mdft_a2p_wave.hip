@@ -8,11 +8,19 @@ namespace mdft {
 
 namespace {
 
-// The points of a field from which a lane per point is faster: half of the CUs
-// have a block (microseconds, mdft_proj.hip's kernel against this one: 8000
-// points FP64 mmax 5 23.4 / 21.4, 13824 mmax 3 15.0 / 12.3, 4096 mmax 5 19.2 /
-// 20.6, mmax 3 7.9 / 9.9).
-constexpr long kMinPoints = 120 * 64;
+// The points of a field from which a lane per point is faster: a block takes 64 of
+// them however few there are, and half of the CUs or more need one.  Microseconds,
+// mdft_proj.hip's kernel against this one:
+//   mmax 5  FP64 5832 points 20.5 / 19.5, 8000 23.3 / 19.4; FP32 8000 19.0 / 15.4
+//   mmax 6  FP64 8000 37.7 / 37.7, 10648 48.6 / 39.2; FP32 5832 23.1 / 24.7, 8000 30.3 / 25.2
+//   mmax 4  FP64 8000 16.1 / 16.7, 10648 18.6 / 16.8; FP32 8000 14.0 / 13.9, 10648 16.1 / 14.4
+//   mmax 3  FP64 8000 9.7 / 9.6 (mrso 1 14.9 / 15.9), 10648 12.2 / 10.3; FP32 8000
+//           8.4 / 9.1 (mrso 1 12.6 / 13.0), 10648 9.6 / 8.7
+//   mmax 2  FP64 8000 7.6 / 8.3 (mrso 1 9.9 / 10.4), 10648 9.1 / 8.8; FP32 13824
+//           7.5 / 7.7 (mrso 1 9.3 / 9.9), 17576 9.3 / 8.7
+long min_points(int mmax, bool fp64) {
+  return mmax >= 5 ? 7680 : mmax > 2 || fp64 ? 10240 : 16384;
+}
 
 // A block takes 64 consecutive r, one per lane, and its waves share out the
 // projections.  For each theta the 64 rows of (phi, psi) values go through LDS
@@ -246,7 +254,7 @@ __global__ __launch_bounds__((64 * A2pPlan<MMAX, MRSO, CP>().waves)) void angl2p
 template <typename TI, typename TP, typename TC>
 bool launch_a2p_wave(const ProjTables& t, long N, long field, const TI* o, cplx<TP>* p, const TabPtrs<TC>& tb,
                      const double* drho_rho0, hipStream_t s, bool compact) {
-  if (field < kMinPoints) return false;
+  if (field < min_points(t.mmax, std::is_same<TC, double>::value)) return false;
   bool done = false;
   dispatch_angular(t.mmax, t.mrso, [&](auto mm, auto mr) {
     constexpr int MMAX = decltype(mm)::value, MRSO = decltype(mr)::value;
