@@ -271,9 +271,16 @@ __global__ __launch_bounds__(kFftThreads) void fft_axis_kernel(cplx<T>* __restri
   }
 }
 
+// whether a tile of W columns of stride S has a compiled kernel: it may be wider
+// than the stride as long as half of its columns exist (the missing ones are
+// computed on for nothing)
+bool compiled_columns(int n, int W, long S) { return ct_length(n) && strided_lines(W) && 2 * S >= W; }
+
 // default tile: a compiled width where there is one, else about 1024 values
+template <typename T>
 int choose_tile_lines(int n, bool strided) {
-  if (ct_length(n)) return strided ? 16 : contiguous_lines(n);
+  if (strided && ct_length(n)) return 16;
+  if (!strided && ct_length(n)) return contiguous_lines<T>(n);
   int W = 1024 / n;
   if (W < 1) W = 1;
   if (W > 64) W = 64;
@@ -293,15 +300,14 @@ void launch_plane(cplx<T>* data, const FftPlan1D& pz, const FftPlan1D& py, long 
   MDFT_HIP_CHECK(hipGetLastError());
 }
 
-// W = 0: the default tile.  A compiled strided tile may be wider than the
-// stride as long as half of its columns exist (the missing ones are computed on
-// for nothing); with fewer, the run-time kernel takes a tile of the S columns.
+// W = 0: the default tile.  A strided tile wider than the stride that is not
+// compiled is one of the S columns.
 template <typename T>
 void launch_axis(cplx<T>* data, const FftPlan1D& p, int sign, long nlines_or_outer, long S, bool strided,
                  hipStream_t stream, int W = 0) {
   if (p.st.n == 1 || nlines_or_outer == 0) return;
-  if (W <= 0) W = choose_tile_lines(p.st.n, strided);
-  if (strided && S < W && !(ct_length(p.st.n) && strided_lines(W) && 2 * S >= W)) W = static_cast<int>(S);
+  if (W <= 0) W = choose_tile_lines<T>(p.st.n, strided);
+  if (strided && S < W && !compiled_columns(p.st.n, W, S)) W = static_cast<int>(S);
   const size_t lds = axis_lds<T>(p.st.n, W);
   throw_if(lds > kLdsMax, "FFT tile does not fit in LDS");
   const cplx<T>* tw = p.twiddles<T>();
@@ -409,9 +415,8 @@ void Fft3dPlan::execute(cplx<T>* data, long batch, int sign, hipStream_t stream)
 }
 
 // Times the candidate configurations on a scratch array of `batch`
-// transforms and keeps the fastest: the tile width of each per-axis pass (16 or
-// 32 columns of the compiled kernels, 256, 512, 1024 or 2048 values per tile of
-// the run-time ones) and, where a (y, z) plane fits in
+// transforms and keeps the fastest: the tile width of each per-axis pass (the
+// compiled ones, else 256, 512, 1024 or 2048 values per tile of the run-time kernel) and, where a (y, z) plane fits in
 // LDS, the fused z/y pass with 256 or 512 threads.  Every candidate runs the
 // same Stockham stages on the same lines, so the choice changes timing only.
 template <typename T>
@@ -446,8 +451,12 @@ FftConfig Fft3dPlan::autotune(long batch, hipStream_t s) const {
     const long nxl = nx, nyl = ny, nzl = nz;
     // per-axis tile widths: the compiled ones, else tiles of 256 .. 2048 values
     auto candidates = [](int n, long S, bool strided) {
-      if (ct_length(n)) return strided ? std::vector<int>{16, 32} : std::vector<int>{contiguous_lines(n)};
       std::vector<int> w;
+      if (!strided && ct_length(n)) w.push_back(contiguous_lines<T>(n));
+      if (strided)
+        for (int W : {16, 32})
+          if (compiled_columns(n, W, S)) w.push_back(W);
+      if (!w.empty()) return w;
       for (int vals : {256, 512, 1024, 2048}) {
         w.push_back(std::max(1, std::min(64, vals / std::max(1, n))));
         if (strided && S < w.back()) w.back() = static_cast<int>(S);

@@ -142,14 +142,19 @@ constexpr int ct_radix(int s) {
     }
   return 0;
 }
-// lines per tile: of the contiguous axis about 1024 values; of a strided axis
-// 16 or 32 neighbouring columns (whole 128-byte lines in FP32, and a tile of a
-// few KB at every length), whether they divide the stride or not: a last tile
-// with missing columns costs one part in the number of tiles, while a width that
-// had to divide the stride left 48^2 and 96^2 to the run-time kernel (4 x 48^3:
-// 175 us for the x axis alone, now 97).
-constexpr int contiguous_lines(int n) { return n <= 16 ? 64 : 1024 / n; }
-inline bool strided_lines(int w) { return w == 16 || w == 32; }
+// Lines per tile of the contiguous axis: 8 KB of values, and at most 64 (one pass
+// over 73 x 64^3 values, us, tiles of 4 / 8 / 16 KB: FP32 64-long lines 43 / 38 /
+// 39, 45 53 / 48 / 55, 96 56 / 49 / 57; FP64 64 86 (8) / 88 (16), 45 100 / 130, 96 102 / 132).
+template <typename T>
+constexpr int contiguous_lines(int n) {
+  const int w = 8192 / static_cast<int>(sizeof(cplx<T>)) / n;
+  return w < 64 ? w : 64;
+}
+// Tiles of a strided axis: 16 or 32 neighbouring columns, whether they divide the
+// stride or not: a last tile with missing columns costs one part in the number
+// of tiles, while a width that had to divide it left 48^2 and 96^2 to the
+// run-time kernel (4 x 48^3: 175 us for the x axis alone, now 97).
+constexpr bool strided_lines(int w) { return w == 16 || w == 32; }
 
 template <typename T, int R, int N, int NS, int LS, int ES, int NLINES, int NTH, bool W_FAST>
 __device__ __forceinline__ void ct_stage_2d(const cplx<T>* src, cplx<T>* dst, const cplx<T>* tw, int sign, int tid) {
@@ -288,12 +293,15 @@ __global__ __launch_bounds__(NTH) void fft_plane_ct_kernel(cplx<T>* __restrict__
   }
 }
 
-// fft_axis_kernel for length N and tiles of W lines (the last tile of a row of
-// tiles may be ragged: its missing lines are computed on and not stored)
+// fft_axis_kernel for length N and tiles of W lines, nchunk of them in a strided
+// row of S columns.  The last tile may be ragged: its missing lines are computed
+// on and not stored.  Whole tiles have a branch of their own, whose loads are
+// requested together: a test of each value against the end of the data took
+// the 64-long FP64 lines of 73 x 64^3 values from 86 to 113 us, FP32 from 38 to 42.
 template <typename T, bool STRIDED, int N, int W>
 __global__ __launch_bounds__(kFftThreads) void fft_axis_ct_kernel(cplx<T>* __restrict__ data,
                                                                   const cplx<T>* __restrict__ tw_g, int sign,
-                                                                  long nlines, long S) {
+                                                                  long nlines, long S, unsigned nchunk) {
   extern __shared__ unsigned char lds_raw[];
   constexpr int LD = N + 1, NTH = kFftThreads, WN = W * N, ITERS = (WN + NTH - 1) / NTH;
   cplx<T>* bufA = reinterpret_cast<cplx<T>*>(lds_raw);
@@ -302,46 +310,51 @@ __global__ __launch_bounds__(kFftThreads) void fft_axis_ct_kernel(cplx<T>* __res
   const int tid = threadIdx.x;
   if (tid < N) tw[tid] = tw_g[tid];
   long base;
-  int valid;  // lines of this tile (STRIDED), or its values
+  int valid;  // lines of this tile
   if constexpr (!STRIDED) {
     const long l0 = static_cast<long>(blockIdx.x) * W;
     base = l0 * N;
-    valid = static_cast<int>(min(static_cast<long>(W), nlines - l0)) * N;
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      if (t < valid) bufA[(t / N) * LD + t % N] = data[base + t];
-    }
+    valid = static_cast<int>(min(static_cast<long>(W), nlines - l0));
   } else {
-    const long nchunk = (S + W - 1) / W;
-    const long o = blockIdx.x / nchunk, i0 = (blockIdx.x - o * nchunk) * W;
-    base = o * N * S + i0;
+    const unsigned o = blockIdx.x / nchunk;
+    const long i0 = static_cast<long>(blockIdx.x - o * nchunk) * W;
+    base = static_cast<long>(o) * N * S + i0;
     valid = static_cast<int>(min(static_cast<long>(W), S - i0));
-    if (tid % W < valid) {
+  }
+  // value i of this thread: its place in the tile's data, and in LDS
+  const auto from = [&](int i) {
+    const int t = tid + i * NTH;
+    return base + (STRIDED ? static_cast<long>(t / W) * S + t % W : t);
+  };
+  const auto to = [&](int i) {
+    const int t = tid + i * NTH;
+    return STRIDED ? (t % W) * LD + t / W : (t / N) * LD + t % N;
+  };
+  const auto in_tile = [&](int i) { return WN % NTH == 0 || tid + i * NTH < WN; };
+  const auto exists = [&](int i) {
+    const int t = tid + i * NTH;
+    return in_tile(i) && (STRIDED ? t % W : t / N) < valid;
+  };
+  if (valid == W) {
 #pragma unroll
-      for (int i = 0; i < ITERS; ++i) {
-        const int t = tid + i * NTH;
-        const int e = t / W, w = t % W;
-        if (WN % NTH == 0 || t < WN) bufA[w * LD + e] = data[base + static_cast<long>(e) * S + w];
-      }
-    }
+    for (int i = 0; i < ITERS; ++i)
+      if (in_tile(i)) bufA[to(i)] = data[from(i)];
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < ITERS; ++i)
+      if (exists(i)) bufA[to(i)] = data[from(i)];
   }
   __syncthreads();
   ct_stockham_2d<T, N, LD, 1, W, NTH, false>(bufA, bufB, tw, sign, tid);
   const cplx<T>* res = ct_nstages<N>() % 2 == 0 ? bufA : bufB;
-  if constexpr (!STRIDED) {
+  if (valid == W) {
 #pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      if (t < valid) data[base + t] = res[(t / N) * LD + t % N];
-    }
-  } else if (tid % W < valid) {
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int t = tid + i * NTH;
-      const int e = t / W, w = t % W;
-      if (WN % NTH == 0 || t < WN) data[base + static_cast<long>(e) * S + w] = res[w * LD + e];
-    }
+    for (int i = 0; i < ITERS; ++i)
+      if (in_tile(i)) data[from(i)] = res[to(i)];
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < ITERS; ++i)
+      if (exists(i)) data[from(i)] = res[to(i)];
   }
 }
 
@@ -369,19 +382,24 @@ bool launch_axis_ct(cplx<T>* data, const cplx<T>* tw, int n, int W, bool strided
   bool done = false;
   for_length(n, CtLengths{}, [&](auto nn) {
     constexpr int N = decltype(nn)::value;
-    auto go = [&](auto kernel, int w, long nblk) {
+    auto go = [&](auto kernel, int w, long nchunk) {
+      const long nblk = strided ? nlines_or_outer * nchunk : nchunk;
       throw_if(nblk > 0x7fffffffL, "too many FFT tiles");
       hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nblk)), dim3(kFftThreads), axis_lds<T>(N, w), stream, data,
-                         tw, sign, nlines_or_outer, S);
+                         tw, sign, nlines_or_outer, S, static_cast<unsigned>(nchunk));
       MDFT_HIP_CHECK(hipGetLastError());
       done = true;
     };
     if (!strided) {
-      constexpr int w = contiguous_lines(N);
+      constexpr int w = contiguous_lines<T>(N);
       if (W == w) go(fft_axis_ct_kernel<T, false, N, w>, w, (nlines_or_outer + w - 1) / w);
     } else {
-      if (W == 16) go(fft_axis_ct_kernel<T, true, N, 16>, 16, nlines_or_outer * ((S + 15) / 16));
-      if (W == 32) go(fft_axis_ct_kernel<T, true, N, 32>, 32, nlines_or_outer * ((S + 31) / 32));
+      auto columns = [&](auto ww) {
+        constexpr int w = decltype(ww)::value;
+        if (W == w) go(fft_axis_ct_kernel<T, true, N, w>, w, (S + w - 1) / w);
+      };
+      columns(std::integral_constant<int, 16>{});
+      columns(std::integral_constant<int, 32>{});
     }
   });
   return done;
