@@ -274,12 +274,21 @@ __global__ __launch_bounds__(kFftThreads) void fft_axis_kernel(cplx<T>* __restri
 // whether a tile of W columns of stride S has a compiled kernel: it may be wider
 // than the stride as long as half of its columns exist (the missing ones are
 // computed on for nothing)
-bool compiled_columns(int n, int W, long S) { return ct_length(n) && strided_lines(W) && 2 * S >= W; }
+bool compiled_columns(int n, int W, long S) { return ct_length(n) && strided_lines(n, W) && 2 * S >= W; }
 
-// default tile: a compiled width where there is one, else about 1024 values
+// default tile: a compiled width where there is one, else about 1024 values.
+// Strided axes of compiled lengths: 16 columns, 32 or 64 of short lines; 8 of long
+// ones where 16 would leave a CU fewer than 7 tiles (1168 x 128 x 16 FP32 27 us
+// against 22, 389 x 96 x 64 27 / 25, but with 8 times the tiles 84 / 104 and
+// 82 / 110); no more than it takes for a thin stride.
 template <typename T>
-int choose_tile_lines(int n, bool strided) {
-  if (strided && ct_length(n)) return 16;
+int choose_tile_lines(int n, bool strided, long outer, long S) {
+  if (strided && ct_length(n)) {
+    int W = n <= 16 ? 64 : n <= 32 ? 32 : 16;
+    if (n > 64 && outer * ((S + 15) / 16) < 7 * 256) W = 8;
+    while (W / 2 >= S && strided_lines(n, W / 2)) W /= 2;
+    return W;
+  }
   if (!strided && ct_length(n)) return contiguous_lines<T>(n);
   int W = 1024 / n;
   if (W < 1) W = 1;
@@ -306,7 +315,7 @@ template <typename T>
 void launch_axis(cplx<T>* data, const FftPlan1D& p, int sign, long nlines_or_outer, long S, bool strided,
                  hipStream_t stream, int W = 0) {
   if (p.st.n == 1 || nlines_or_outer == 0) return;
-  if (W <= 0) W = choose_tile_lines<T>(p.st.n, strided);
+  if (W <= 0) W = choose_tile_lines<T>(p.st.n, strided, nlines_or_outer, S);
   if (strided && S < W && !compiled_columns(p.st.n, W, S)) W = static_cast<int>(S);
   const size_t lds = axis_lds<T>(p.st.n, W);
   throw_if(lds > kLdsMax, "FFT tile does not fit in LDS");
@@ -454,8 +463,8 @@ FftConfig Fft3dPlan::autotune(long batch, hipStream_t s) const {
       std::vector<int> w;
       if (!strided && ct_length(n)) w.push_back(contiguous_lines<T>(n));
       if (strided)
-        for (int W : {16, 32})
-          if (compiled_columns(n, W, S)) w.push_back(W);
+        for (int W : {4, 8, 16, 32, 64})
+          if (compiled_columns(n, W, S) && (W > 4 || S < 8)) w.push_back(W);
       if (!w.empty()) return w;
       for (int vals : {256, 512, 1024, 2048}) {
         w.push_back(std::max(1, std::min(64, vals / std::max(1, n))));

@@ -150,11 +150,16 @@ constexpr int contiguous_lines(int n) {
   const int w = 8192 / static_cast<int>(sizeof(cplx<T>)) / n;
   return w < 64 ? w : 64;
 }
-// Tiles of a strided axis: 16 or 32 neighbouring columns, whether they divide the
-// stride or not: a last tile with missing columns costs one part in the number
-// of tiles, while a width that had to divide it left 48^2 and 96^2 to the
-// run-time kernel (4 x 48^3: 175 us for the x axis alone, now 97).
-constexpr bool strided_lines(int w) { return w == 16 || w == 32; }
+// Tiles of a strided axis: 16 neighbouring columns and, for short lines, 32 or 64,
+// for long ones 8, which some fields need to fill the chip (9 x 128 x 32 x 64
+// FP32, y and x: 16 columns 38 us, 8 37; 1168 x 128 x 16 27.6 against 22.3), and 4
+// (strides below 8).  They need not divide the stride: a last tile with missing
+// columns costs one part in the number of tiles, while a width that had to
+// divide it left 48^2 and 96^2 to the run-time kernel (4 x 48^3: 175 us for the
+// x axis alone, now 97).
+constexpr bool strided_lines(int n, int w) {
+  return w == 16 || (w == 32 && n <= 64) || (w == 64 && n <= 32) || ((w == 4 || w == 8) && n >= 64);
+}
 
 template <typename T, int R, int N, int NS, int LS, int ES, int NLINES, int NTH, bool W_FAST>
 __device__ __forceinline__ void ct_stage_2d(const cplx<T>* src, cplx<T>* dst, const cplx<T>* tw, int sign, int tid) {
@@ -396,10 +401,14 @@ bool launch_axis_ct(cplx<T>* data, const cplx<T>* tw, int n, int W, bool strided
     } else {
       auto columns = [&](auto ww) {
         constexpr int w = decltype(ww)::value;
-        if (W == w) go(fft_axis_ct_kernel<T, true, N, w>, w, (S + w - 1) / w);
+        if constexpr (strided_lines(N, w))
+          if (W == w) go(fft_axis_ct_kernel<T, true, N, w>, w, (S + w - 1) / w);
       };
+      columns(std::integral_constant<int, 4>{});
+      columns(std::integral_constant<int, 8>{});
       columns(std::integral_constant<int, 16>{});
       columns(std::integral_constant<int, 32>{});
+      columns(std::integral_constant<int, 64>{});
     }
   });
   return done;
