@@ -409,11 +409,11 @@ void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, in
 
 template <typename T>
 FftConfig Fft3dPlan::default_config() const {
+  const bool compiled = ny == nz && plane_ct(ny, sizeof(cplx<T>));
   FftConfig c;
   c.plane = plane_ok(sizeof(cplx<T>)) &&
-            (ny == nz && plane_ct(ny, sizeof(cplx<T>)) ? plane_ct_bytes(ny, sizeof(cplx<T>)) : plane_lds<T>(ny, nz)) <=
-                kPlaneLdsMax;
-  c.plane_threads = 512;
+            (compiled ? plane_ct_bytes(ny, sizeof(cplx<T>)) : plane_lds<T>(ny, nz)) <= kPlaneLdsMax;
+  c.plane_threads = compiled ? plane_ct_threads(ny, 512) : 512;
   return c;
 }
 
@@ -497,6 +497,7 @@ FftConfig Fft3dPlan::autotune(long batch, hipStream_t s) const {
     float best_t = z.second + y.second + x.second;
     if (plane_ok(sizeof(cplx<T>)) && batch * nxl <= 0x7fffffffL) {
       for (int th : {256, 512}) {
+        if (ny == nz && plane_ct(ny, sizeof(cplx<T>)) && plane_ct_threads(ny, th) != th) continue;
         FftConfig c = axes;
         c.plane = true;
         c.plane_threads = th;

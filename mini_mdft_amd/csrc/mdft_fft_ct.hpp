@@ -375,8 +375,17 @@ bool launch_axis_ct(cplx<T>* data, const cplx<T>* tw, int n, int W, bool strided
 // whether n x n planes of elem-byte values have a compile-time kernel (n up to
 // 128 in FP32, 100 in FP64)
 inline bool plane_ct(int n, size_t elem) { return ct_length(n) && plane_ct_bytes(n, elem) <= kLdsMax; }
-// launches it, if there is one (the lengths that have one thread count take
-// that one, whatever threads says)
+// The lengths whose planes are compiled with 256 and with 512 threads, for the
+// tuner to choose: the multiples of 16 up to 96.  256 against 512, us for 73 x 64^3
+// values: FP32 16 71 / 112, 32 50 / 55, 48 57 / 58, 64 52 / 53, 80 73 / 77, 96 89 /
+// 84; FP64 16 118 / 181, 32 99 / 97, 48 100 / 106, 64 200 / 105, 80 211 / 204, 96
+// 293 / 212.  The others have one count: up to 32 a stage has at most 256
+// butterflies of radix 4 and a block of 512 would idle; above, 512 threads keep
+// eight waves on a CU where only one or two planes fit in its LDS.
+constexpr bool both_threads(int n) { return n % 16 == 0 && n <= 96; }
+// the threads a plane of compiled length n runs with if `threads` are asked for
+constexpr int plane_ct_threads(int n, int threads) { return both_threads(n) ? threads : n <= 32 ? 256 : 512; }
+// launches it with plane_ct_threads(n, threads), if there is one
 template <typename T>
 bool launch_plane_ct(cplx<T>* data, const cplx<T>* tw, int n, long planes, int threads, int sign, hipStream_t s);
 

@@ -10,13 +10,6 @@ template <typename T, int N>
 constexpr bool plane_fits() {
   return plane_ct_bytes(N, sizeof(cplx<T>)) <= kLdsMax;
 }
-// The lengths whose planes are compiled with 256 and with 512 threads (the
-// tuner's choice).  The others have one count: up to 32 a stage has at most 256
-// butterflies of radix 4 and a block of 512 would idle; above, 512 threads keep
-// eight waves on a CU where only one or two planes fit in its LDS.
-constexpr bool both_threads(int n) {
-  return n == 16 || n == 32 || n == 48 || n == 64 || n == 80 || n == 96;
-}
 
 }  // namespace
 
@@ -38,7 +31,7 @@ bool launch_plane_ct(cplx<T>* data, const cplx<T>* tw, int n, long planes, int t
         else
           go(fft_plane_ct_kernel<T, N, 512>, 512);
       } else {
-        constexpr int th = N <= 32 ? 256 : 512;
+        constexpr int th = plane_ct_threads(N, 0);
         go(fft_plane_ct_kernel<T, N, th>, th);
       }
     }
