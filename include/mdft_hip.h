@@ -135,12 +135,14 @@ int mdft_fft3d(void* data, int batch, int nx, int ny, int nz, int sign, int dtyp
 
 /* The same transform in a given configuration (no counterpart in the
  * reference): plane != 0 runs z and y as one pass over each (y, z) plane
- * staged in LDS (plane_threads 256 or 512; radices 2-5; the plane must fit in
- * 160 KB of LDS), else one pass per axis with wz / wy / wx lines per tile
- * (0: the default).  Every configuration runs the same butterflies on the
- * same lines: results are bitwise those of mdft_fft3d.  A Convolution tunes
- * its configuration on first use by timing these candidates;
- * mdft_conv_fft_config reports it (tuned = 0 before the first execute). */
+ * staged in LDS (plane_threads 256 or 512; the plane must be square with a side
+ * of 8 .. 128 (dtype MDFT_DOUBLE: 100), or have radices 2-5 and fit twice in
+ * 160 KB of LDS), else one pass per axis with wz / wy / wx lines per tile (0:
+ * the default; a width without a compiled kernel takes the slower run-time
+ * one).  Every configuration runs the same butterflies on the same lines:
+ * results are bitwise those of mdft_fft3d.  A Convolution tunes its
+ * configuration on first use by timing candidates; mdft_conv_fft_config reports
+ * it (tuned = 0 before the first execute), and it may be given here. */
 int mdft_fft3d_config(void* data, int batch, int nx, int ny, int nz, int sign, int dtype, int plane,
                       int plane_threads, int wz, int wy, int wx, void* stream);
 int mdft_conv_fft_config(mdft_conv_t h, int* tuned, int* plane, int* plane_threads, int* wz, int* wy, int* wx);

@@ -419,8 +419,6 @@ int mdft_fft3d_config(void* data, int batch, int nx, int ny, int nz, int sign, i
     c.wz = wz;
     c.wy = wy;
     c.wx = wx;
-    throw_if(c.plane && !plan.plane_run_time(dtype == MDFT_DOUBLE ? 16 : 8),
-             "FFT: the fused plane pass does not apply to this shape");
     hipStream_t s = as_stream(stream);
     if (dtype == MDFT_DOUBLE)
       plan.execute_config<double>(c, static_cast<cplx<double>*>(data), batch, sign, s);

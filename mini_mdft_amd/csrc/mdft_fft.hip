@@ -382,12 +382,11 @@ const cplx<float>* FftPlan1D::twiddles<float>() const {
 
 Fft3dPlan::Fft3dPlan(int nx_, int ny_, int nz_) : nx(nx_), ny(ny_), nz(nz_), px(nx_), py(ny_), pz(nz_) {}
 
-bool Fft3dPlan::plane_run_time(size_t elem) const {
+bool Fft3dPlan::plane_ok(size_t elem) const {
+  if (ny == nz && plane_ct(ny, elem)) return true;
   return ny > 1 && nz > 1 && small_radices(py.st) && small_radices(pz.st) &&
          (2 * static_cast<size_t>(ny) * (nz + 1) + ny + nz) * elem <= kLdsMax;
 }
-
-bool Fft3dPlan::plane_ok(size_t elem) const { return (ny == nz && plane_ct(ny, elem)) || plane_run_time(elem); }
 
 template <typename T>
 void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, int sign, hipStream_t stream) const {

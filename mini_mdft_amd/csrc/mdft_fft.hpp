@@ -58,9 +58,8 @@ struct Fft3dPlan {
   FftConfig default_config() const;
   template <typename T>
   bool tuned() const { return tuned_[std::is_same<T, double>::value ? 1 : 0]; }
+  // whether a kernel takes z and y planes of elem-byte values in one pass
   bool plane_ok(size_t elem) const;
-  // whether the run-time plane kernel takes them
-  bool plane_run_time(size_t elem) const;
 
  private:
   mutable FftConfig cfg_[2];
