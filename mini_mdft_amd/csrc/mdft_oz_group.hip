@@ -695,12 +695,26 @@ int place(int e) {
 
 }  // namespace
 
+// A group of stars costs a CU the same however many of its stars exist, and a
+// round of groups the chip: at mmax 5 12 us + 11.5 us a round of 8 stars per CU,
+// where the star kernel takes 13 us + 6.9 ns a star.  So the last round decides
+// (star kernel against this one, 2048 stars a round, FP32, us):
+//   2197 stars 27.6 / 35.6, 2744 30.8 / 35.4, 3375 35.4 / 35.3, 3640 38.4 / 35.1,
+//   4096 40.1 / 35.2, 4356 42.9 / 45.8, 4807 44.4 / 45.9, 4913 46.4 / 46.4,
+//   5265 45.7 / 45.9, 6859 59.4 / 57.5, 9261 76.0 / 68.8, 15625 128 / 103
+// and this kernel is taken where its rounds are filled to 0.82.  At mmax 4, whose
+// stars are half as large and whose blocks share a CU, the sides meet at 17576
+// stars (78.9 / 78.3; 15625 65.7 / 71.2, 19305 88.2 / 86.2, 21021 93.5 / 93.9,
+// 24389 110 / 102, 35937 180 / 148).
 bool OzGroup::serves(int mmax, int mrso, long nstars) {
-  // mmax 5: 47.7 against 49.1 us at 32^3 (4913 stars), 36.7 against 29.0 at
-  // 24^3; mmax 4, whose stars are half as large: 102 against 110 us at 56^3
-  // (24 389 stars), 72.5 against 71.3 at 48^3
   if (mrso != 2) return false;
-  return mmax == 5 ? nstars >= 4900 : mmax == 4 ? nstars >= 20000 : false;
+  if (mmax == 4) return nstars >= 19000;
+  if (mmax != 5) return false;
+  int dev = 0, cus = 0;
+  MDFT_HIP_CHECK(hipGetDevice(&dev));
+  MDFT_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const long round = static_cast<long>(kStars) * std::max(1, cus), rounds = (nstars + round - 1) / round;
+  return 100 * nstars >= 82 * rounds * round;
 }
 
 OzGroup::OzGroup(const ConvTables& tab, hipStream_t s)
