@@ -309,9 +309,9 @@ __device__ __forceinline__ double inverse_distance(double d2) {
 // FP64 arithmetic bounds it, and a pair alone costs 31 vector operations, 15 of
 // them the minimum image and 10 the reciprocal root; the tile shares the x term
 // of d^2 over its nodes, the y terms over its columns and the z terms over its
-// rows, so that a pair has one addition and the root left.  A call at 64^3 /
-// mmax 5 with 20 x 2 pairs: one node 3228 us, 2 x 2 2309, 2 x 4 2006, 4 x 4 1927,
-// 4 x 8 (256 registers, one wave per SIMD) slower again.  The sums are the ones
+// rows, so that a pair has one addition and the root left: 64^3 / mmax 5 with 20
+// x 2 pairs 3042 us with one node and 1744 with 4 x 4 (kVextCost; 4 x 8, with 256
+// registers and one wave per SIMD, is slower again).  The sums are the ones
 // vext_site makes, product for product.  Missing nodes of a ragged tile
 // repeat the last node and are not stored.
 template <int TY, int TZ, bool BOUNDED>
@@ -406,6 +406,47 @@ constexpr double kPi = 3.14159265358979323846;
 const double kQfact = kQunit * kQunit * 1.0e-3 * kNavo / (4.0 * kPi * kEps0 * 1.0e-10);
 
 
+// Tiles of 1, 2 or 4 nodes along y and z: us of a call at 64^3 / mmax 5 with 20 x 2
+// pairs, 50 of them the host's, taken off.
+constexpr int kVextCost[3][3] = {{2990, 2450, 2120}, {2540, 1985, 1765}, {2260, 1815, 1685}};
+
+struct VextTile {
+  int y, z;  // log2 of the nodes
+};
+
+// The tile whose cost, with the nodes that it computes past the end of a row or
+// column for nothing, is least: 4 x 4 alone took 510 us for 128 x 128 x 1, where 4
+// x 1 takes 258 and one node 308, and 217 against 196 (2 x 2) for 96 x 9 x 9.  Up
+// to 16 nodes where that leaves every CU a block, else 4 (16^3, mmax 4, 58k
+// against 230k threads: 108 and 106 us a call; 8^3, mmax 3, 76 and 59).
+VextTile vext_tile(int ny, int nz, long n) {
+  VextTile best{0, 0};
+  double least = 0.0;
+  for (int y = 0; y < 3; ++y)
+    for (int z = 0; z < 3; ++z) {
+      if (y + z > (n / 16 < 65536 ? 2 : 4)) continue;
+      const long rows = (ny + (1 << y) - 1) >> y << y, columns = (nz + (1 << z) - 1) >> z << z;
+      const double cost = static_cast<double>(kVextCost[y][z]) * rows * columns;
+      if (least == 0.0 || cost < least) {
+        least = cost;
+        best = {y, z};
+      }
+    }
+  return best;
+}
+
+// launch(kernel, nodes along y, along z) of a tile
+template <int Y = 0, int Z = 0, typename F>
+void launch_vext_tile(VextTile t, F&& launch) {
+  if (t.y == Y && t.z == Z) {
+    launch(vext_kernel<1 << Y, 1 << Z, true>, 1 << Y, 1 << Z);
+  } else if constexpr (Z < 2) {
+    launch_vext_tile<Y, Z + 1>(t, launch);
+  } else if constexpr (Y < 2) {
+    launch_vext_tile<Y + 1, 0>(t, launch);
+  }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -499,20 +540,16 @@ void compute_vext(int nx, int ny, int nz, double lx, double ly, double lz, const
     hipLaunchKernelGGL(kernel, dim3(grid_for(threads, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin, dvr,
                        doff, dpair, dpos, vext);
   };
-  // 16 nodes per thread where that leaves every CU a block, else 4 (16^3, mmax
-  // 4, 58k against 230k threads: 117 and 115 us a call; 30 x 42 x 27, mmax 3,
-  // 191k: 102 and 109).  inverse_distance needs a finite d^2; coordinates that
-  // could overflow it keep the library's root.
+  // inverse_distance needs a finite d^2; coordinates that could overflow it keep
+  // the library's root
   auto bounded = [](const double* v, size_t count) {
     return std::all_of(v, v + count, [](double x) { return std::abs(x) <= 1e100; });
   };
   const double box[3] = {lx, ly, lz};
   if (!bounded(box, 3) || !bounded(pos.data(), pos.size()) || !bounded(off.data(), off.size()))
     launch(vext_kernel<2, 2, false>, 2, 2);
-  else if (n / 16 < 65536)
-    launch(vext_kernel<2, 2, true>, 2, 2);
   else
-    launch(vext_kernel<4, 4, true>, 4, 4);
+    launch_vext_tile(vext_tile(ny, nz, n), launch);
   MDFT_HIP_CHECK(hipGetLastError());
   // the tables (host and device) are released on return
   MDFT_HIP_CHECK(hipStreamSynchronize(s));
