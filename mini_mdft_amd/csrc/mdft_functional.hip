@@ -292,8 +292,9 @@ __device__ __forceinline__ double site_coordinate(int i, double h, double o) {
 }
 
 // min(1 / d, 1e6) from d^2.  BOUNDED (d^2 < inf): the hardware's estimate y and
-// one third-order step, y (1 - e)^(-1/2) = y (1 + e/2 + 3 e^2 / 8 + ..) with
-// e = 1 - d^2 y^2 (d = 0: NaN, which the minimum takes to 1e6).  Against
+// one third-order Householder step for y^(-2) = d^2, the binomial series y (1 -
+// e)^(-1/2) = y (1 + e/2 + 3 e^2 / 8 + ..) with e = 1 - d^2 y^2 (d = 0: NaN, which
+// the minimum takes to 1e6).  Against
 // rsqrt(), which also selects for 0 and infinity: 2167 -> 1927 us at 64^3 / mmax
 // 5 with 20 x 2 pairs, the same bits.
 template <bool BOUNDED>
@@ -540,13 +541,13 @@ void compute_vext(int nx, int ny, int nz, double lx, double ly, double lz, const
     hipLaunchKernelGGL(kernel, dim3(grid_for(threads, kFThreads, 65536)), dim3(kFThreads), 0, s, a, origin, dvr,
                        doff, dpair, dpos, vext);
   };
-  // inverse_distance needs a finite d^2; coordinates that could overflow it keep
-  // the library's root
+  // inverse_distance needs a finite d^2; coordinates that could overflow it, or
+  // whose quotient by a side could, keep the library's root
   auto bounded = [](const double* v, size_t count) {
     return std::all_of(v, v + count, [](double x) { return std::abs(x) <= 1e100; });
   };
   const double box[3] = {lx, ly, lz};
-  if (!bounded(box, 3) || !bounded(pos.data(), pos.size()) || !bounded(off.data(), off.size()))
+  if (!bounded(box, 3) || std::min({lx, ly, lz}) < 1e-100 || !bounded(pos.data(), pos.size()) || !bounded(off.data(), off.size()))
     launch(vext_kernel<2, 2, false>, 2, 2);
   else
     launch_vext_tile(vext_tile(ny, nz, n), launch);

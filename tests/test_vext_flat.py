@@ -32,3 +32,12 @@ def test_tiles(oracle, sides, values):
     # rounding of the sum: some 1e-16 of its largest terms, which the cap bounds
     # only from above
     assert np.abs(V - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.gpu
+def test_side_without_a_quotient():
+    """A box of 1e-309 A, whose reciprocal overflows: d^2 is infinite, 1/d is 0."""
+    n, L = (2, 3, 3), (1e-309,) * 3
+    sol = np.array([[1.0, 0.0, 0.0, 3.0, 2.0, 1.0]])
+    V = M.vext(M.SpatialGrid(n, L), M.AngularGrid(2, 2), sol, SOLV[1:2], 300.0).cpu().numpy()
+    assert (V == 0.0).all()
