@@ -591,11 +591,11 @@ __global__ __launch_bounds__(kThreads) void delta_f_kernel(const T* __restrict__
 }
 
 // block j: out[j out_stride] = scale * sum of partials[j count .. (j + 1) count)
-// in a fixed order: thread t sums t, t + T, ... in four interleaved chains,
-// then the block combines the threads' sums as a tree.  One block, so its time
-// is the latency of its loads: up to 32 of a thread are in flight together (a
-// round of four at a time 9.1 us at 64^3 mmax 5, 24576 partials and 5280 extra
-// terms)
+// in a fixed order: thread t sums t, t + T, ... in four interleaved chains (all
+// four loads of a round in flight together), then the block combines the
+// threads' sums as a tree.  Rounds of 8, 12, 24 or 32 loads, whose code is longer,
+// are no faster (24576 partials 6.4 us, 7.2 to 7.6 with them, 6.5 with 24; 82944
+// partials and 5280 extra terms 17.4, 18.9 to 19.4)
 constexpr int kRedThreads = 1024;
 __global__ __launch_bounds__(kRedThreads) void reduce_partials_kernel(const double* __restrict__ partials, int count,
                                                                       double scale, double* __restrict__ out,
@@ -607,37 +607,16 @@ __global__ __launch_bounds__(kRedThreads) void reduce_partials_kernel(const doub
   constexpr int T = kRedThreads;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
   int i = threadIdx.x;
-  // rounds of one value per chain, R of them with their loads in flight together
-  const auto rounds = [&](auto rr) {
-    constexpr int R = decltype(rr)::value;
-    for (; i + (4 * R - 1) * T < count; i += 4 * R * T) {
-      double v[4 * R];
-#pragma unroll
-      for (int u = 0; u < 4 * R; ++u) v[u] = partials[i + u * T];
-#pragma unroll
-      for (int u = 0; u < 4 * R; u += 4) {
-        a0 += v[u];
-        a1 += v[u + 1];
-        a2 += v[u + 2];
-        a3 += v[u + 3];
-      }
-    }
-  };
-  rounds(std::integral_constant<int, 8>{});
-  rounds(std::integral_constant<int, 3>{});
-  rounds(std::integral_constant<int, 1>{});
-  for (; i < count; i += T) a0 += partials[i];
-  if (extra) {  // the extra terms of this field, after the partials, in the same fixed order
-    const double* from = extra + static_cast<long>(blockIdx.x) * nextra;
-    for (int e0 = threadIdx.x; e0 < nextra; e0 += 8 * T) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = from[min(e0 + u * T, nextra - 1)];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (e0 + u * T < nextra) a1 += v[u];
-    }
+  for (; i + 3 * T < count; i += 4 * T) {
+    const double v0 = partials[i], v1 = partials[i + T], v2 = partials[i + 2 * T], v3 = partials[i + 3 * T];
+    a0 += v0;
+    a1 += v1;
+    a2 += v2;
+    a3 += v3;
   }
+  for (; i < count; i += T) a0 += partials[i];
+  if (extra)  // the extra terms of this field, after the partials, in the same fixed order
+    for (int e = threadIdx.x; e < nextra; e += T) a1 += extra[static_cast<long>(blockIdx.x) * nextra + e];
   __shared__ double red[T];
   red[threadIdx.x] = (a0 + a1) + (a2 + a3);
   __syncthreads();
