@@ -39,14 +39,23 @@ namespace mdft {
 namespace {
 
 // The sum of column col of nin rows, rows c kFan .. (fixed order; rows past the
-// last read as zero), all kFan loads in flight together.
+// last read as zero), all kFan loads in flight together.  A whole set of rows has
+// a branch without a test per row: 8.7 -> 6.6 us of the first pass at 64^3 mmax 5,
+// and 9.6 -> 4.8 of the gemv kernel below, whose rows are whole there.
 constexpr int kFan = 64;
 __device__ __forceinline__ double column_sum(const double* __restrict__ src, long nin, int width, long c, int col) {
   double v[kFan];
+  src += c * kFan * width + col;
+  const int rows = static_cast<int>(min(static_cast<long>(kFan), nin - c * kFan));
+  if (rows == kFan) {
 #pragma unroll
-  for (int i = 0; i < kFan; ++i) v[i] = src[min(c * kFan + i, nin - 1) * width + col];
+    for (int i = 0; i < kFan; ++i) v[i] = src[static_cast<long>(i) * width];
+  } else {
 #pragma unroll
-  for (int i = 0; i < kFan; ++i) v[i] = c * kFan + i < nin ? v[i] : 0.0;
+    for (int i = 0; i < kFan; ++i) v[i] = src[static_cast<long>(min(i, rows - 1)) * width];
+#pragma unroll
+    for (int i = 0; i < kFan; ++i) v[i] = i < rows ? v[i] : 0.0;
+  }
 #pragma unroll
   for (int h = kFan / 2; h > 0; h >>= 1)
 #pragma unroll
