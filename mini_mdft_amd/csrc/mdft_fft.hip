@@ -398,7 +398,7 @@ void Fft3dPlan::execute_config(const FftConfig& c, cplx<T>* data, long batch, in
                  (c.plane_threads != 256 && c.plane_threads != 512),
              "FFT: the fused plane pass does not apply to this shape");
     // z and y in one pass over each contiguous (y, z) plane
-    launch_plane<T>(data, pz, py, planes, c.plane_threads, sign, stream);
+    if (planes > 0) launch_plane<T>(data, pz, py, planes, c.plane_threads, sign, stream);
   } else {
     launch_axis<T>(data, pz, sign, batch * nxl * nyl, 1, false, stream, c.wz);  // z: contiguous lines
     launch_axis<T>(data, py, sign, batch * nxl, nzl, true, stream, c.wy);       // y: stride nz

@@ -70,3 +70,13 @@ def test_reported_configuration_is_accepted(n, prec):
     M.fft3d_config(y, -1, bool(c.pop("plane")), **c)
     M.fft3d(ref, -1)
     assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("n", [64, 96, 100])
+@pytest.mark.parametrize("dt", [0, 1])
+def test_no_transforms(n, dt):
+    """A batch of none is done, in planes as in axis passes."""
+    from mini_mdft_amd._lib import check, lib
+
+    x = torch.zeros(1, dtype=torch.complex128, device="cuda")
+    check(lib().mdft_fft3d(x.data_ptr(), 0, 2, n, n, -1, dt, None))
