@@ -20,7 +20,8 @@
 // re, im, -q re, im) of one pair and writes them with one or two wide stores.
 // v_mfma_f32_16x16x4_f32 accumulates its four products as sequential FMAs in
 // the order of K: the sums run in the order of the one-output-per-thread
-// kernels, bit for bit where c is real.
+// kernels, bit for bit where c is real (ten grids of 600 to 36 000 stars with
+// both kernels, in both channel orders).
 //
 // What bounds the pass.  Per star it moves 2 x 8 x np values and does 209
 // kflop at mmax 5, 140 MFMA tiles: 4480 cycles of a SIMD, 70 us for the
@@ -38,7 +39,7 @@
 //   * each star belongs to one wave, so that the three products need no
 //     barrier between them; a wave requests all operands of a step before its
 //     first product.
-// 64^3, mmax 5: 334 -> 229 us (80^3: 576 -> 397, 96^3: 961 -> 685); two waves
+// 64^3, mmax 5: 334 -> 217 us (80^3: 576 -> 399, 96^3: 961 -> 685 to 705); two waves
 // per SIMD (LDS holds 8 stars of 19 KB) leave the OZ product at about half of
 // the matrix rate.  Measured and left out: 4-wave blocks of 4 stars, two per CU
 // (276 us), two waves per star (spills at 128 registers: 424 us), and FP64 (4
