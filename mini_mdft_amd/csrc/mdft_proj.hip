@@ -424,7 +424,7 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
   const long base = r0 * A::kNo + th * A::kNjk;
   // The phi and psi sums and the epilogue.  A generic lambda, whose loops unroll
   // before it is inlined: written into the kernel itself they left 127 registers
-  // at mmax 6 and few projections in flight (X6F, 64^3: 1443 us against 752).
+  // at mmax 6 and few projections in flight (X6F, 64^3: 1443 us where this took 752).
   const auto outputs = [&](auto first) {
     constexpr int j0 = decltype(first)::value;
     TC* out = stage + lane * W;
@@ -462,26 +462,27 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
       // xi^2 - 1 and of vexc build up in registers (each row's W values are
       // one contiguous run of xi and df; this walk also measured faster than
       // the row-major one below, 0.358 against 0.371 ms at 64^3).  A row of
-      // mmax 6 has 91 values: a second walk takes the columns from 64 on (staged
-      // and walked in two halves instead, the sums and both walks took 340
-      // registers: X6F, 64^3, 1075 us against 752)
+      // mmax 6 has 91 values: a second walk takes the 27 from 64 on, two rows at
+      // a time, one per half wave (X6F, 64^3: 677 us; a row at a time 752; staged
+      // and walked in two halves, whose sums and walks took 340 registers, 1075)
       constexpr int kRB = 32;  // rows per batch of loads in flight
       const int nrow = static_cast<int>(min(static_cast<long>(kWaveRows), N - r0));
 #pragma unroll
       for (int w0 = 0; w0 < W; w0 += 64) {
-        const bool on = W - w0 >= 64 || w0 + lane < W;
-        const int jk = W - w0 >= 64 ? w0 + lane : min(w0 + lane, W - 1);
+        const int per = w0 > 0 && W - w0 <= 32 ? 2 : 1, sub = per == 2 ? lane >> 5 : 0, col = per == 2 ? lane & 31 : lane;
+        const bool on = W - w0 >= 64 || w0 + col < W;
+        const int jk = W - w0 >= 64 ? w0 + col : min(w0 + col, W - 1);
         double cs = 0.0, cv = 0.0;
-        for (int rl0 = 0; rl0 < kWaveRows; rl0 += kRB) {
+        for (int rl0 = 0; rl0 < kWaveRows; rl0 += kRB * per) {
           double xv[kRB];
 #pragma unroll
           for (int b = 0; b < kRB; ++b) {
-            const int rl = min(rl0 + b, nrow - 1);
+            const int rl = min(rl0 + b * per + sub, nrow - 1);
             xv[b] = static_cast<double>(xi[base + static_cast<long>(rl) * A::kNo + jk]);
           }
 #pragma unroll
           for (int b = 0; b < kRB; ++b) {
-            const int rl = rl0 + b;
+            const int rl = rl0 + b * per + sub;
             if (on && rl < nrow) {
               const double x = xv[b];
               const double vx = static_cast<double>(static_cast<TO>(stage[rl * W + jk]));
@@ -493,7 +494,11 @@ __global__ __launch_bounds__(64) void proj2angl_wave_kernel(const cplx<TP>* __re
             }
           }
         }
-        if (on) {
+        if (per == 2) {
+          cs += __shfl_xor(cs, 32);
+          cv += __shfl_xor(cv, 32);
+        }
+        if (on && sub == 0) {
           // colpart[rb][0][io] = sum_r (xi^2 - 1), colpart[rb][1][io] = sum_r vexc
           double* cp = colpart + rb * (2 * A::kNo) + th * A::kNjk + jk;
           cp[0] = cs;
